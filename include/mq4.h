@@ -179,7 +179,7 @@ int mq4_rmsnorm_gate_up_silu(const uint16_t* x, int64_t M, int64_t K,
  * SwiGLU epilogue writes h so.  With every scale and bias row 16-byte
  * aligned the products use fp16 weights (fp16(s q + b), about 2e-6 of the
  * output rms from the exact product) on an fp16 copy of the operands, and
- * the down product runs in 1, 2 or 4 K parts whose fp32 sums go to the
+ * the down product runs in 1 to 6 K parts whose fp32 sums go to the
  * workspace and are added in order with the residual; otherwise the exact
  * bf16 operands with their group sums.  From 5 to 32 rows
  * (with 64 < N / 64 <= 96) the down product runs as two halves of K per

@@ -142,50 +142,35 @@ __device__ __forceinline__ uint32_t swiglu_bf16(float g_acc, float u_acc) {
     return f32_to_bf16(t * u);
 }
 
-// swiglu_bf16 of N (gate, up) pairs through a table of the rounded SiLU
-// t(g) = round_bf16(round_bf16(1 / (1 + expf(-g))) * g), the same bits.  The
-// table holds t for the bf16 g with 2^-9 <= |g| < 128 (exponent fields
-// 118-133; entry (sign << 11) | (exponent - 118) << 7 | mantissa, 4096 x 2
-// bytes, silu_lut_entry).  Below 2^-9 the rounded sigmoid is 0.5 exactly, so
-// t = g / 2: the exponent field less one for exponent fields 2-117, and
-// +-0 for +-0.  The rest (|g| >= 128, inf, NaN, and |g| < 2^-125 where g / 2
-// is subnormal) take the exact formula, in one branch for the batch.
+// swiglu_bf16 of N (gate, up) pairs through a table of the rounded sigmoid
+// s(g) = round_bf16(1 / (1 + expf(-g))) of the bf16 gate value, the same
+// bits.  The table holds s for the bf16 g with 2^-9 <= |g| < 128 (exponent
+// fields 118-133; entry (sign << 11) | (exponent - 118) << 7 | mantissa, 4096
+// x 2 bytes, silu_lut_entry).  |g| is clamped to that range: s(+-2^-9) is
+// 0.5, as it is for every smaller |g|; beyond 127.5 it is 1 or 0, as at 127.5
+// (expf(-g) is 0 or infinite from |g| = 104 on).  NaN gates get some s of the
+// table and stay NaN in s * g.
 constexpr int SILU_LUT_N = 4096;
-constexpr uint32_t SILU_LUT_LO = 118u << 7;          // |g| bits of 2^-9
+constexpr uint32_t SILU_LUT_LO = 118u << 7;       // |g| bits of 2^-9
 __device__ __forceinline__ uint32_t silu_lut_entry(uint32_t i) {
 #pragma clang fp contract(off)
     const uint32_t bits = ((i >> 11) << 15) | (SILU_LUT_LO + (i & 2047u));
-    const float g = bf16_to_f32(bits);
-    return f32_to_bf16(round_bf16(1.0f / (1.0f + expf(-g))) * g);
+    return f32_to_bf16(1.0f / (1.0f + expf(-bf16_to_f32(bits))));
 }
 template <int N>
 __device__ __forceinline__ void swiglu_bf16_lut_batch(const float (&g_acc)[N], const float (&u_acc)[N],
                                                       uint32_t (&out)[N], const uint16_t* lut) {
 #pragma clang fp contract(off)
-    static_assert(N <= 32, "one mask word");
-    uint32_t gb[N], tb[N];
-    uint32_t need = 0;
+    float g[N], sg[N];
 #pragma unroll
     for (int e = 0; e < N; ++e) {
-        gb[e] = f32_to_bf16(g_acc[e]);
-        const uint32_t mag = gb[e] & 0x7fffu;
-        const uint32_t k = mag - SILU_LUT_LO;                            // unsigned
-        const uint32_t idx = (k < 2048u ? k : 0u) | ((gb[e] >> 4) & 0x800u);
-        const uint32_t lt = lut[idx];
-        const bool half = mag - 0x100u < SILU_LUT_LO - 0x100u;           // exponent fields 2-117
-        tb[e] = k < 2048u ? lt : half ? gb[e] - 0x80u : gb[e];           // +-0 keeps its bits
-        if (k >= 2048u && !half && mag != 0u) need |= 1u << e;
-    }
-    if (need) {
-#pragma unroll
-        for (int e = 0; e < N; ++e)
-            if (need & (1u << e)) {
-                const float g = bf16_to_f32(gb[e]);
-                tb[e] = f32_to_bf16(round_bf16(1.0f / (1.0f + expf(-g))) * g);
-            }
+        g[e] = round_bf16(g_acc[e]);
+        const float m = __builtin_amdgcn_fmed3f(fabsf(g[e]), 0x1p-9f, 127.5f);
+        const uint32_t idx = ((__float_as_uint(m) >> 16) - SILU_LUT_LO) | ((__float_as_uint(g[e]) >> 20) & 0x800u);
+        sg[e] = bf16_to_f32(lut[idx & (SILU_LUT_N - 1)]);
     }
 #pragma unroll
-    for (int e = 0; e < N; ++e) out[e] = f32_to_bf16(bf16_to_f32(tb[e]) * round_bf16(u_acc[e]));
+    for (int e = 0; e < N; ++e) out[e] = f32_to_bf16(round_bf16(sg[e] * g[e]) * round_bf16(u_acc[e]));
 }
 
 // Monotone 16-bit key of a bf16 value for max-selection: larger value ->

@@ -39,12 +39,12 @@ struct GemmArgs {
 int launch_q4_gemm(const GemmArgs& a, int epi, bool norm, hipStream_t st);
 
 // The fp16-weight GEMM (mq4_gemm16.hip): x holds fp16 activations in the
-// operand order of launch_pair_rows16, row m scaled by 1 / (xscale[m] *
+// operand order of launch_pair_rows16 (by k group: [K / 64][M][64]), row m scaled by 1 / (xscale[m] *
 // ascale) (xscale null: 1; ascale 0: 1), and the product of row m is
 // multiplied back by xscale[m] * ascale (powers of two).  Epilogues
 // GEMM_RESIDUAL and GEMM_SWIGLU as GemmArgs, plus:
-//  * GEMM_SWIGLU with yscale != 0: y = fp16(h * yscale) in the operand order
-//    (h the bf16 SwiGLU value; saturated at +-65504), no ysum; with
+//  * GEMM_SWIGLU with yscale != 0: y = fp16(h * yscale) in the operand order,
+//    by group as x (h the bf16 SwiGLU value; saturated at +-65504), no ysum; with
 //    yscale == 0 and ysum: the bf16 paired h and its group sums (N % 128 ==
 //    0), as GemmArgs.
 struct Gemm16Args {
@@ -57,15 +57,13 @@ struct Gemm16Args {
     float* ysum;
     float ascale;            // a power of two, or 0 (1)
     float yscale;            // GEMM_SWIGLU: fp16 output scale, or 0 (bf16 output)
-    // GEMM_RESIDUAL in 1 < ksplit <= 4 K parts (K / 64 a multiple of 8 ksplit):
-    // part[k][M][N] fp32 (16-byte aligned, N % 4 == 0), then a second kernel
-    // adds the parts in order and the residual (res and y 8-byte aligned)
+    // GEMM_RESIDUAL in 1 < ksplit <= 6 K parts (gemm16_parts; 1 is always
+    // possible): part[k][M][N] fp32 (16-byte aligned, N % 4 == 0), then a
+    // second kernel adds the parts in order and the residual (res and y
+    // 8-byte aligned)
     int ksplit;
     float* part;
-    // GEMM_RESIDUAL: nonzero for blocks of 128 weight columns (one 32-column
-    // MFMA tile per wave, three blocks per CU) instead of 256; the same bits
-    int narrow;
-    // GEMM_SWIGLU: the 4096-entry SiLU table of silu_lut_entry (16-byte
+    // GEMM_SWIGLU: the SiLU's 4096-entry sigmoid table, silu_lut_entry (16-byte
     // aligned; launch_pair_rows16 writes it)
     const uint16_t* silu_lut;
 };
@@ -76,8 +74,12 @@ struct Gemm16Args {
 // bits).
 int launch_q4_gemm16(const Gemm16Args& a, int epi, hipStream_t st);
 
+// K parts of the fp16-weight GEMM_RESIDUAL product of this shape (K % 512 ==
+// 0); changes with M at multiples of 64 only, and past 128 rows never grows.
+int gemm16_parts(int64_t M, int64_t N, int64_t K);
+
 // xp = fp16(x / xscale[m]) (norm_w null) or fp16(bf16(x * rsqrt(mean(x^2) +
-// eps) * (1 + norm_w)) / xscale[m]) in the operand order (the bits of
+// eps) * (1 + norm_w)) / xscale[m]) in the operand order, by k group (the bits of
 // mq4_rms_norm before the conversion), with xscale[m] = 2^e, e >= 0 the
 // smallest that keeps the row below 2^15.  K % 512 == 0; x, xp, norm_w
 // 16-byte aligned.  silu_lut non-null: the same launch also writes the

@@ -32,27 +32,33 @@
 // fp16 is subnormal: an absolute error under 2^-25 of the row's scale.
 //
 // Work decomposition:
-//  * A 256-thread block computes 128 rows x 256 weight columns (one matrix:
-//    256 output columns; gate and up: 128 output columns each, for the fused
-//    SwiGLU); wave w takes all 128 rows and 64 weight columns (gate/up:
-//    32 gate and the same 32 up columns) as 4 x 2 v_mfma_f32_32x32x16_f16
-//    tiles, so each weight is dequantized once per block, by the one wave
-//    that uses it (about two VALU per weight: a v_and_or_b32 forms two fp16
-//    1024 + q, a v_pk_add_f16 takes the 1024 off, a v_pk_fma_f16 applies s
-//    and b to the pair).
-//  * Per 64-k group, the 128 x 64 activations (16 KB, each row's eight
-//    16-byte chunks XOR-swizzled by (row / 2) % 8: the 16 lanes of a
-//    ds_read_b128 phase, 16 rows at one chunk, cover the 64 banks once) and
-//    the 256 x 32 bytes of packed weights (per 32 columns one DMA
-//    instruction, lane l reading k-half l / 32 of column l % 32, so that the
-//    stage holds each k-half's 32 columns in consecutive slots) go to LDS by
-//    DMA, two stages, one group ahead;
-//    the columns' scales and biases follow every eight groups (16 bytes per
-//    column, two slots).  Each step waits for all of its wave's DMA;
-//    barriers carry no memory fence.  (Per-group DMA of the scales, four
-//    bytes from 64 columns per instruction, and of one k-half of 64 columns
-//    made the kernel bound by L2 requests: 17.5 M per gate/up call at M =
-//    2048.)
+//  * A wave takes 32 RI rows and 64 weight columns (gate/up: 32 gate and the
+//    same 32 up columns) as RI x 2 v_mfma_f32_32x32x16_f16 tiles and
+//    dequantizes its own weights: 13 VALU per packed word of eight (a
+//    v_and_or_b32 forms two fp16 1024 + q, a v_pk_add_f16 takes the 1024 off,
+//    a v_pk_fma_f16 applies s and b to the pair, one shift per word).  What a
+//    wave issues bounds it: 112 VALU per k group against 8 RI MFMAs of 14 ns
+//    (one wave per SIMD issues a VALU every 2.4 ns, two waves one every
+//    2.0 ns, MFMAs of either wave running beside them), so RI = 4 wherever
+//    the rows fill it, and as little else in the loop as possible: 8 groups
+//    unrolled, every LDS address a constant, scales and biases read once per
+//    8 groups.
+//  * The ring and the schedule are in gemm16_tile, the tile shapes and the
+//    rule that picks one in tile_for.  At full load (M = 8192) the card holds
+//    the clock at 1.8 GHz (2.6 GHz with few blocks) and MFMAs are busy 57% of
+//    the cycles, as in a large library product (59% at 2.15 GHz): power, not
+//    a unit, is the bound there.
+//  * Per 64-k group, the activations (each row's eight 16-byte chunks
+//    XOR-swizzled by (row / 2) % 8: the 16 lanes of a ds_read_b128 phase, 16
+//    rows at one chunk, cover the 64 banks once) and the packed weights (per
+//    32 columns one DMA instruction, lane l reading k-half l / 32 of column
+//    l % 32, so that the stage holds each k-half's 32 columns in consecutive
+//    slots) go to LDS by DMA; the columns' scales and biases follow every
+//    eight groups (16 bytes per column, two slots).  Barriers carry no memory
+//    fence.  (Per-group DMA of the scales, four bytes from 64 columns per
+//    instruction, made the kernel bound by L2 requests.)
+//  * Activations are stored by k group, [group][row][64], so that a tile's
+//    group is one contiguous run.
 //  * The operand layout is mq4_gemm.hip's: lane l of a tile holds row (or
 //    weight column) l % 32 and k-half l / 32; MFMA step ks takes word ks of
 //    the half, whose nibble pairs (q_p, q_{p+4}) meet the activations in the
@@ -60,15 +66,14 @@
 //    row operand and the activations its column operand, so that a result
 //    lane holds one activation row and four runs of four consecutive weight
 //    columns: the epilogue reads one row scale per 32 rows and writes 8-byte
-//    runs.  (With the activations as the row operand a lane held one column
-//    of 16 rows: a row-scale load and a 2-byte store per output, which cost
-//    the SwiGLU product 26 us of 72 at M = 2048 in a copy without the
-//    dequantization and the data movement.)
+//    runs.
 #include <type_traits>
 
 #include "mq4_device.h"
 #include "mq4_gemm.h"
+#include "mq4_gemv.h"
 #include "mq4_host.h"
+#include "mq4_stage.h"
 
 namespace mq4 {
 
@@ -76,46 +81,57 @@ namespace g16 {
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kNW = 4;                    // waves per block
-constexpr int kThreads = 64 * kNW;
-constexpr int TBM = 128;                  // rows per block
-constexpr int A_I = TBM * 8 / (64 * kNW); // activation DMA instructions per wave and group (4)
+constexpr int NJ = 2;                     // 32-column MFMA tiles per wave (SwiGLU: a gate and an up tile)
 
-// NJ 32-column MFMA tiles per wave: a block covers BNW = 32 NJ kNW weight
-// columns (NJ = 2: 256, two blocks per CU; NJ = 1: 128, three blocks per CU).
-template <int NJ>
-struct Cols {
-    static constexpr int BNW = 32 * NJ * kNW;          // weight columns per block
-    static constexpr int B_I = 2 * BNW / 64 / kNW;     // weight DMA instructions per wave and group (NJ)
-    static constexpr int SB_I = 2 * BNW / (64 * kNW);  // scale/bias DMA instructions per wave and 8 groups (NJ)
+// A block of KW teams of WR x WC waves, each wave 32 RI rows x 64 weight
+// columns; the teams compute the same tile over their own parts of K.
+template <int WR, int WC, int RI, int KW>
+struct Shape {
+    static constexpr int NW = WR * WC, THREADS = 64 * NW * KW;
+    static constexpr int TBM = 32 * RI * WR;            // rows per block
+    static constexpr int BNW = 32 * NJ * WC;            // weight columns per block
+    static constexpr int A_I = TBM / 8 / NW;            // activation DMA instructions per wave and group
+    static constexpr int B_I = BNW / 32 / NW;           // weight DMA instructions per wave and group
+    static constexpr int SB_I = 2 * BNW / 64 / NW;      // scale/bias DMA instructions per wave and 8 groups
+    static constexpr int LUT_I = SILU_LUT_N / 512 / (NW * KW); // SiLU table DMA instructions per wave
+    static_assert(A_I * 8 * NW == TBM && B_I * 32 * NW == BNW && SB_I * 64 * NW == 2 * BNW &&
+                      LUT_I * 512 * NW * KW == SILU_LUT_N,
+                  "every wave issues the same DMA");
 };
 
-template <int NJ>
+// One k group: activations [row][chunk ^ ((row >> 1) & 7)] (fp16 pairs) and
+// packed weights [32-column block][k-half][column].
+template <int TBM, int BNW>
 struct Stage {
-    uint4 a[TBM * 8];                     // [row][chunk ^ ((row >> 1) & 7)], fp16 pairs
-    uint4 b[2 * Cols<NJ>::BNW];           // [32-column block][k-half][column]
+    uint4 a[TBM * 8];
+    uint4 b[2 * BNW];
 };
-// Scales and biases of 8 groups: [scales | biases][weight column], 16 bytes
-// (groups 8 t .. 8 t + 7) each.
-template <int NJ>
-struct SbStage {
-    uint4 v[2][Cols<NJ>::BNW];
+// A team's ring: S stages; scales and biases of 8 groups, [scales |
+// biases][weight column], 16 bytes (groups 8 t .. 8 t + 7) each, two slots.
+template <int TBM, int BNW, int S>
+struct Ring {
+    Stage<TBM, BNW> st[S];
+    uint4 sb[2][2][BNW];
 };
-static_assert(2 * sizeof(Stage<2>) + 2 * sizeof(SbStage<2>) <= 65536, "LDS DMA targets must lie in the first 64 KiB");
-static_assert(3 * (2 * sizeof(Stage<1>) + 2 * sizeof(SbStage<1>)) <= 160 * 1024, "three NJ = 1 blocks per CU");
+template <int EPI, int TBM, int BNW, int S, int KW>
+struct Smem {
+    Ring<TBM, BNW, S> ring[KW];
+    __align__(16) uint16_t lut[EPI == GEMM_SWIGLU ? SILU_LUT_N : 8];
+};
 
-__device__ __forceinline__ void lds_dma16(const void* src, void* lds) {
-    __builtin_amdgcn_global_load_lds(src, lds, 16, 0, 0);
-}
-__device__ __forceinline__ void lds_dma4(const void* src, void* lds) {
-    __builtin_amdgcn_global_load_lds(src, lds, 4, 0, 0);
+// A bf16 value (its float bits) as a pair of the same fp16 (round to nearest
+// even; exact for bf16 values of fp16's normal range).
+__device__ __forceinline__ h2_t bf16_to_h2(uint32_t float_bits) {
+    const _Float16 v = (_Float16)__uint_as_float(float_bits);
+    return (h2_t){v, v};
 }
 
-// bf16 bits -> fp16 (round to nearest even; exact for bf16 values of fp16's
-// normal range)
-__device__ __forceinline__ _Float16 bf16_to_h(uint32_t bits) { return (_Float16)bf16_to_f32(bits); }
+__device__ __forceinline__ uint32_t word_of(const uint4& v, int i) {
+    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
+}
 
 // (s & m) | c in one v_and_or_b32, the mask in an SGPR and the exponent
 // bits in a VGPR, both set up once by the caller: the nibbles m selects in
@@ -160,70 +176,39 @@ __device__ __forceinline__ void mfma_result_pad() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int EPI, int NJ>
-__global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Gemm16Args p) {
+// One block's tile: rows m0 .. m0 + TBM - 1, weight columns of n0 .., K part
+// kpart of S_K (split again over the block's KW teams).
+template <int EPI, int WR, int WC, int RI, int S, int KW, class Sm>
+__device__ __forceinline__ void gemm16_tile(const Gemm16Args& p, Sm& smem_all, int n0, int m0, int kpart, int S_K) {
 #pragma clang fp contract(off)
+    using Sh = Shape<WR, WC, RI, KW>;
     static_assert(EPI == GEMM_SWIGLU || EPI == GEMM_RESIDUAL, "the epilogues of mq4_mlp_residual");
-    static_assert(NJ == 2 || (NJ == 1 && EPI == GEMM_RESIDUAL), "SwiGLU: a gate and an up tile per wave");
     constexpr int NMAT = EPI == GEMM_SWIGLU ? 2 : 1;
-    constexpr int BNW = Cols<NJ>::BNW, B_I = Cols<NJ>::B_I, SB_I = Cols<NJ>::SB_I;
+    constexpr int TBM = Sh::TBM, BNW = Sh::BNW, A_I = Sh::A_I, B_I = Sh::B_I, SB_I = Sh::SB_I;
     constexpr int BN = BNW / NMAT;                       // output columns per block
-    using Stage = g16::Stage<NJ>;
-    using SbStage = g16::SbStage<NJ>;
-    // one LDS object, stages first: the DMA targets stay in the first 64 KiB
-    // (SwiGLU: the 8 KB SiLU table after them, read only by the epilogue)
-    struct Smem {
-        Stage st[2];
-        SbStage sb[2];
-        uint16_t lut[EPI == GEMM_SWIGLU ? SILU_LUT_N : 2];
-    };
-    __shared__ Smem smem;
-    Stage &st0 = smem.st[0], &st1 = smem.st[1];
-    SbStage &sb0 = smem.sb[0], &sb1 = smem.sb[1];
-    static_assert(2 * sizeof(Stage) + 2 * sizeof(SbStage) <= 65536, "LDS DMA targets in the first 64 KiB");
+    constexpr int D = A_I + B_I;                         // DMA instructions per wave and stage
+    static_assert((S == 2 || S == 4) && D * (S - 1) < 64, "ring depth");
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int team = bwave / Sh::NW, wave = bwave % Sh::NW;
+    const int wr_ = wave / WC, wc = wave % WC;           // wave row and wave column of the block
     const int h = lane >> 5, col = lane & 31;
     const int M = p.M, N = p.N, K = p.K, G = K / 64;
-    // K parts (GEMM_RESIDUAL): block b takes part b / tiles, groups
-    // [part GL, (part + 1) GL), and writes its fp32 partial product
-    const int S = EPI == GEMM_RESIDUAL && p.ksplit > 1 ? p.ksplit : 1;
-    const int GL = G / S;
-    int bt = blockIdx.x, kpart = 0;
-    if (S > 1) {
-        const int tiles = (int)gridDim.x / S;
-        kpart = bt / tiles;
-        bt -= kpart * tiles;
-    }
+    const int GL = G / (S_K * KW), g0 = (kpart * KW + team) * GL;   // this team's groups g0 .. g0 + GL - 1
+    auto& smem = smem_all.ring[team];
 
-    // XCD-aware block order: with the column blocks a multiple of 8, XCD x
-    // (block b runs on XCD b % 8) takes a fixed eighth of them for every row
-    // block, so its weights stay in its own L2
-    const int NB = (N + BN - 1) / BN;
-    int nb, mb;
-    {
-        const int b = bt;
-        if ((NB & 7) == 0) {
-            const int per = NB >> 3, s = b >> 3;
-            nb = (s % per) * 8 + (b & 7);
-            mb = s / per;
-        } else {
-            nb = b % NB;
-            mb = b / NB;
-        }
-    }
-    const int n0 = nb * BN, m0 = mb * TBM;
-
-    // ---- DMA sources: wave-uniform bases plus 32-bit lane byte offsets ----
-    const char* const xbase = reinterpret_cast<const char*>(p.x) + (int64_t)kpart * GL * 128;
+    // ---- DMA sources: wave-uniform pointers, moved along K one group per
+    // step, plus 32-bit lane byte offsets ----
+    const int64_t xg = (int64_t)M * 128;               // bytes of one group's rows
+    const char* xp = reinterpret_cast<const char*>(p.x) + g0 * xg;
     uint32_t aoff[A_I];
 #pragma unroll
     for (int t = 0; t < A_I; ++t) {
         const int slot = (wave * A_I + t) * 64 + lane;
         const int r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
         const int row = (m0 + r) < M ? (m0 + r) : (M - 1);
-        aoff[t] = (uint32_t)(((int64_t)row * K + c * 8) * 2);
+        aoff[t] = (uint32_t)(row * 128 + c * 16);
     }
     // weight column r of the block -> matrix and output row (rows past N
     // repeat row N - 1, never stored)
@@ -236,32 +221,45 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
     // k-half l / 32 of column l % 32 (its group's 32 bytes as two 16-byte
     // halves), so the stage holds [32-column block][k-half][column] and the
     // operand reads of a k-half are 32 consecutive 16-byte slots
-    const char* bbase[B_I];
+    const char* bp[B_I];
     uint32_t boff[B_I];
 #pragma unroll
     for (int t = 0; t < B_I; ++t) {
         const int r0 = (wave * B_I + t) * 32;
-        bbase[t] = reinterpret_cast<const char*>(mat_of(r0).wq) + (int64_t)kpart * GL * 32;
+        bp[t] = reinterpret_cast<const char*>(mat_of(r0).wq) + (int64_t)g0 * 32;
         boff[t] = (uint32_t)((int64_t)wrow_of(r0 + (lane & 31)) * (K / 2) + (lane >> 5) * 16);
     }
     // scales and biases: 16 bytes (8 groups) of one weight column per lane
-    const char* sbbase[SB_I];
+    const char* sbp[SB_I];
     uint32_t sboff[SB_I];
 #pragma unroll
     for (int t = 0; t < SB_I; ++t) {
         const int u0 = (wave * SB_I + t) * 64, sel = u0 / BNW, r0 = u0 % BNW;
-        sbbase[t] = reinterpret_cast<const char*>(sel ? mat_of(r0).b : mat_of(r0).s) + (int64_t)kpart * (GL / 8) * 16;
+        sbp[t] = reinterpret_cast<const char*>(sel ? mat_of(r0).b : mat_of(r0).s) + (int64_t)(g0 / 8) * 16;
         sboff[t] = (uint32_t)((int64_t)wrow_of(r0 + lane) * G * 2);
     }
-    auto issue = [&](int g, Stage& st) {
+    // LDS byte addresses of this wave's DMA blocks in stage 0 and slot 0
+    const uint32_t a_lds = stage::lds_addr(&smem.st[0].a[0]) + (uint32_t)(wave * A_I * 1024);
+    const uint32_t b_lds = stage::lds_addr(&smem.st[0].b[0]) + (uint32_t)(wave * B_I * 1024);
+    const uint32_t sb_lds = stage::lds_addr(&smem.sb[0][0][0]) + (uint32_t)(wave * SB_I * 1024);
+    constexpr uint32_t STG = sizeof(smem.st[0]), SBS = sizeof(smem.sb[0]);
+    // the group xp / bp point at -> ring stage `slot`; then the pointers move
+    // on by `step` groups (0 at the end of K: the last group again)
+    auto issue = [&](int slot, int step) {
 #pragma unroll
-        for (int t = 0; t < A_I; ++t) lds_dma16(xbase + g * 128 + aoff[t], &st.a[(wave * A_I + t) * 64]);
+        for (int t = 0; t < A_I; ++t) stage::dma16_m0(xp, aoff[t], a_lds + slot * STG + t * 1024);
 #pragma unroll
-        for (int t = 0; t < B_I; ++t) lds_dma16(bbase[t] + g * 32 + boff[t], &st.b[(wave * B_I + t) * 64]);
+        for (int t = 0; t < B_I; ++t) stage::dma16_m0(bp[t], boff[t], b_lds + slot * STG + t * 1024);
+        xp += step * xg;
+#pragma unroll
+        for (int t = 0; t < B_I; ++t) bp[t] += step * 32;
     };
-    auto issue_sb = [&](int t8, SbStage& sbs) {        // groups 8 t8 .. 8 t8 + 7
+    auto issue_sb = [&](uint32_t slot, int step) {     // the next eight groups' scales and biases
 #pragma unroll
-        for (int t = 0; t < SB_I; ++t) lds_dma16(sbbase[t] + t8 * 16 + sboff[t], &sbs.v[0][(wave * SB_I + t) * 64]);
+        for (int t = 0; t < SB_I; ++t) {
+            stage::dma16_m0(sbp[t], sboff[t], sb_lds + slot * SBS + t * 1024);
+            sbp[t] += step * 16;
+        }
     };
 
     // ---- this lane's weight columns (block-relative) of tiles j = 0, 1 ----
@@ -274,7 +272,15 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
     const int ccol = f16_out || paired_out ? ((col & ~7) | perm8(col & 7)) : col;
     int wr[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) wr[j] = NMAT == 2 ? j * (BNW / 2) + wave * 32 + ccol : wave * (32 * NJ) + j * 32 + ccol;
+    for (int j = 0; j < NJ; ++j) wr[j] = NMAT == 2 ? j * (BNW / 2) + wc * 32 + ccol : wc * (32 * NJ) + j * 32 + ccol;
+    // LDS operand addresses (in uint4) within a stage: activation chunk
+    // 4 h + ks of row wr_ RI 32 + col (row tile i: + 256 i), packed words of
+    // column wr[j]
+    uint32_t arow[4], brow[NJ];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) arow[ks] = (uint32_t)((wr_ * RI * 32 + col) * 8 + ((4 * h + ks) ^ ((col >> 1) & 7)));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) brow[j] = (uint32_t)((wr[j] >> 5) * 64 + h * 32 + (wr[j] & 31));
 
     uint32_t nib_mask, nib_exp, nib_mask_hi, nib_exp_hi;   // the nibble-pair constants, set up once
     asm("s_mov_b32 %0, 0x000f000f" : "=s"(nib_mask));
@@ -282,170 +288,222 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
     asm("s_mov_b32 %0, 0x00f000f0" : "=s"(nib_mask_hi));
     asm("v_mov_b32 %0, 0x54005400" : "=v"(nib_exp_hi));
 
-    f32x16_t acc[4][NJ];
+    f32x16_t acc[RI][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < RI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-    // this group's packed words, scales and biases (read before the step's
-    // DMA is issued, so no wait for it can come between)
-    struct Wts {
-        uint4 bw[NJ];
-        h2_t s2[NJ], b2[NJ];
+    uint4 bw[NJ];                                      // a group's packed words
+    uint4 sv[NJ], bv[NJ];                              // eight groups' scales and biases
+    h2_t s2[NJ], b2[NJ];                               // a group's, as fp16 pairs
+    auto read_w = [&](int slot) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) bw[j] = smem.st[slot].b[brow[j]];
     };
-    auto load_wts = [&](int g, const Stage& st) -> Wts {
-        Wts w;
-        const SbStage& sbs = ((g >> 3) & 1) ? sb1 : sb0;
-        const int sh16 = (g & 1) * 16, dw = (g >> 1) & 3;
+    auto read_sb = [&](uint32_t slot) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            w.bw[j] = st.b[(wr[j] >> 5) * 64 + h * 32 + (wr[j] & 31)];
-            const _Float16 s = bf16_to_h((reinterpret_cast<const uint32_t*>(&sbs.v[0][wr[j]])[dw] >> sh16) & 0xffffu);
-            const _Float16 b = bf16_to_h((reinterpret_cast<const uint32_t*>(&sbs.v[1][wr[j]])[dw] >> sh16) & 0xffffu);
-            w.s2[j] = (h2_t){s, s};
-            w.b2[j] = (h2_t){b, b};
+            sv[j] = smem.sb[slot][0][wr[j]];
+            bv[j] = smem.sb[slot][1][wr[j]];
         }
-        return w;
+    };
+    auto group_sb = [&](int u) {                       // group u of the eight
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            s2[j] = bf16_to_h2(u & 1 ? word_of(sv[j], u >> 1) & 0xffff0000u : word_of(sv[j], u >> 1) << 16);
+            b2[j] = bf16_to_h2(u & 1 ? word_of(bv[j], u >> 1) & 0xffff0000u : word_of(bv[j], u >> 1) << 16);
+        }
+    };
+    auto read_a = [&](int slot, int ks, h8_t (&a)[RI]) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i) a[i] = __builtin_bit_cast(h8_t, smem.st[slot].a[arow[ks] + 256 * i]);
+    };
+    auto dequant = [&](int ks, h8_t (&bo)[NJ]) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            bo[j] = dequant_word(word_of(bw[j], ks), s2[j], b2[j], nib_mask, nib_exp, nib_mask_hi, nib_exp_hi);
     };
     // The weights are the MFMA row operand and the activations the column
     // operand: result lane l of tile (i, j) holds activation row i 32 + l % 32.
-    // MFMA step ks + 1's activation reads and dequantization are issued
-    // during step ks's MFMAs (two operand sets), one MFMA per LDS read and
-    // four VALU.
-    auto compute = [&](const Wts& wt, const Stage& st) {
-        const uint4* bw = wt.bw;
-        const h2_t* s2 = wt.s2;
-        const h2_t* b2 = wt.b2;
-        auto read_a = [&](int ks, h8_t (&a)[4]) {
+    auto mfmas = [&](const h8_t (&a)[RI], const h8_t (&bo)[NJ]) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = i * 32 + col, ch = 4 * h + ks;
-                a[i] = __builtin_bit_cast(h8_t, st.a[r * 8 + (ch ^ ((r >> 1) & 7))]);
-            }
-        };
-        auto dequant = [&](int ks, h8_t (&bo)[NJ]) {
+        for (int i = 0; i < RI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const uint32_t w = ks == 0 ? bw[j].x : ks == 1 ? bw[j].y : ks == 2 ? bw[j].z : bw[j].w;
-                bo[j] = dequant_word(w, s2[j], b2[j], nib_mask, nib_exp, nib_mask_hi, nib_exp_hi);
-            }
-        };
-        auto mfmas = [&](const h8_t (&a)[4], const h8_t (&bo)[NJ]) {
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bo[j], a[i], acc[i][j], 0, 0, 0);
+    };
+    auto interleave = [] {                             // one LDS read and the dequantization per MFMA
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int m = 0; m < RI * NJ; ++m) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                   // MFMA
+            if (m < RI) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x002, 28 / (RI * NJ), 0);      // VALU
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // ---- prologue: the table, the first scales and S stages in flight ----
+    if constexpr (EPI == GEMM_SWIGLU) {
 #pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bo[j], a[i], acc[i][j], 0, 0, 0);
-        };
-        auto interleave = [] {
+        for (int t = 0; t < Sh::LUT_I; ++t)
+            stage::dma16_m0(p.silu_lut, (uint32_t)((bwave * Sh::LUT_I + t) * 1024 + lane * 16),
+                            stage::lds_addr(smem_all.lut) + (uint32_t)((bwave * Sh::LUT_I + t) * 1024));
+    }
+    const int nblk = GL / 8;                           // eight-group blocks of this K part
+    issue_sb(0, nblk > 1 ? 1 : 0);
 #pragma unroll
-            for (int m = 0; m < 4 * NJ; ++m) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                 // MFMA
-                if (m < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // LDS read
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);                 // VALU
-            }
+    for (int s = 0; s < S; ++s) issue(s, 1);           // GL >= 8 > S
+    wait_vmcnt<D * (S - 1)>();
+    lds_barrier();                                     // stage 0 (and the table) is in for every wave
+    h8_t a0[RI], a1[RI], w0[NJ], w1[NJ];
+    read_w(0);
+    read_sb(0);
+    read_a(0, 0, a0);
+    group_sb(0);
+    dequant(0, w0);
+
+    // Step u of an eight-group block computes its group from stage u % S
+    // (S divides 8: every LDS address in the step is a constant).  MFMA step
+    // ks + 1's activation reads and dequantization are issued during step
+    // ks's MFMAs (two operand sets); before the last MFMA step the waves meet
+    // (each has read all of the stage, and has waited for its own DMA of the
+    // next one), so that during it the next group's operands are read and the
+    // group S ahead goes into the free stage: a step never starts by waiting
+    // for its operands.  Every step issues D DMA instructions (past the end:
+    // the last group again, into a stage that nobody reads), so one constant
+    // vmcnt serves every step; a block's scales and biases go out just before
+    // its first group.
+    for (int t8 = 0; t8 < nblk; ++t8) {
+        const bool more = t8 + 1 < nblk;               // another block follows
+        const int inc = more ? 1 : 0, sb_inc = t8 + 2 < nblk ? 1 : 0;
+        const uint32_t nsb = (uint32_t)(t8 + 1) & 1;
+        auto step = [&](auto uc) {
+            constexpr int u = decltype(uc)::value, cs = u % S, ns = (u + 1) % S;
+            mfmas(a0, w0);
+            read_a(cs, 1, a1);
+            dequant(1, w1);
+            interleave();
+            mfmas(a1, w1);
+            read_a(cs, 2, a0);
+            dequant(2, w0);
+            interleave();
+            mfmas(a0, w0);
+            read_a(cs, 3, a1);
+            dequant(3, w1);
+            interleave();
+            wait_vmcnt<D * (S - 2)>();
+            lds_barrier();
+            read_w(ns);
+            if constexpr (u == 7) read_sb(nsb);        // past the end: stale bytes, not used
+            read_a(ns, 0, a0);
+            issue(cs, u + S + 1 < 8 ? 1 : inc);
+            if constexpr (u == 7 - S) issue_sb(nsb, sb_inc);
+            mfmas(a1, w1);
+            group_sb((u + 1) & 7);
+            dequant(0, w0);
             __builtin_amdgcn_sched_barrier(0);
         };
-        h8_t a0[4], a1[4], w0[NJ], w1[NJ];
-        read_a(0, a0);
-        dequant(0, w0);
-        read_a(1, a1);
-        dequant(1, w1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(a0, w0);
-        read_a(2, a0);
-        dequant(2, w0);
-        interleave();
-        mfmas(a1, w1);
-        read_a(3, a1);
-        dequant(3, w1);
-        interleave();
-        mfmas(a0, w0);
-        mfmas(a1, w1);
-    };
-    // Two stages: step g waits for all of this wave's DMA (group g's), meets
-    // the other waves at the barrier, reads group g's weights, issues group
-    // g + 1 into the stage read in step g - 1 (past the end: the last group
-    // again, into a stage nobody reads), at every eighth group also the next
-    // eight groups' scales and biases into the slot read by the eight groups
-    // before, and computes group g.
-    auto step = [&](int g, const Stage& cur, Stage& nxt) {
-        wait_vmcnt<0>();
-        lds_barrier();                               // group g is in `cur` for every wave
-        const Wts wt = load_wts(g, cur);
-        issue(g + 1 < GL ? g + 1 : g, nxt);          // into the stage read in step g - 1
-        if ((g & 7) == 0 && g + 8 < GL) issue_sb((g >> 3) + 1, ((g >> 3) & 1) ? sb0 : sb1);
-        compute(wt, cur);
-    };
-    // the SiLU table (SwiGLU) is loaded with group 0 and stored to LDS after
-    // its wait; the first step's barrier publishes it
-    uint4 lut0 = make_uint4(0, 0, 0, 0), lut1 = lut0;
-    if (EPI == GEMM_SWIGLU) {
-        static_assert(SILU_LUT_N * 2 == 2 * 16 * kThreads, "two 16-byte pieces of the table per thread");
-        const uint4* src = reinterpret_cast<const uint4*>(p.silu_lut);
-        lut0 = src[tid];
-        lut1 = src[tid + kThreads];
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+        step(std::integral_constant<int, 7>{});
     }
-    issue(0, st0);
-    issue_sb(0, sb0);
-    if (EPI == GEMM_SWIGLU) {
-        wait_vmcnt<0>();
-        uint4* dst = reinterpret_cast<uint4*>(smem.lut);
-        dst[tid] = lut0;
-        dst[tid + kThreads] = lut1;
-    }
-    int g0 = 0;
-    for (; g0 + 2 <= GL; g0 += 2) {
-        step(g0, st0, st1);
-        step(g0 + 1, st1, st0);
-    }
-    if (g0 < GL) step(g0, st0, st1);
     wait_vmcnt<0>();                                 // no DMA outstanding past the loop
     mfma_result_pad();
+
+    // Teams: each takes over OWN of every wave's row tiles, adding the teams'
+    // sums in team order; they travel through LDS (the rings, free now), each
+    // lane's 16 values of a tile as four 16-byte slots.
+    constexpr int OWN = KW <= RI ? RI / KW : 1;
+    auto mine = [&](int i) { return KW == 1 || i / OWN == team; };   // row tiles this wave writes
+    if constexpr (KW > 1) {
+        static_assert(KW >= RI || RI % KW == 0, "whole row tiles per team");
+        constexpr int CAP = KW <= RI ? RI - OWN : RI;  // row tiles a team hands over, at most
+        f32x4_t* ex = reinterpret_cast<f32x4_t*>(&smem_all.ring[0]);
+        static_assert((size_t)KW * Sh::NW * CAP * NJ * 4 * 64 * 16 <= sizeof(smem_all.ring), "exchange area");
+        auto slot = [&](int k, int i) {
+            return (((k * Sh::NW + wave) * CAP + (KW <= RI && i / OWN > k ? i - OWN : i)) * NJ) * 4 * 64 + lane;
+        };
+        lds_barrier();                                 // every wave is done with its ring
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            if (mine(i)) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    ex[slot(team, i) + (j * 4 + q) * 64] = (f32x4_t){acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                                    acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            if (!mine(i)) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int k = 0; k < KW; ++k) {
+                        const f32x4_t own = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                             acc[i][j][4 * q + 3]};
+                        const f32x4_t v = k == i / OWN ? own : ex[slot(k, i) + (j * 4 + q) * 64];
+                        sum = k == 0 ? v : sum + v;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] = sum[r];
+                }
+        }
+    }
 
     // ---- epilogue: result lane l of tile (i, j) holds activation row
     // i 32 + l % 32 and MFMA rows (e / 4) 8 + (l / 32) 4 + e % 4 of tile j:
     // four runs of four consecutive output columns (natural order, or the
     // pair-order positions 4 (l / 32) .. + 3 of an 8-column chunk), each
     // stored as one 8-byte (16 for fp32) write.
-    // SwiGLU with ysum: h also goes to an LDS tile in natural column order,
-    // 64 rows at a time (stage 0, free once every wave is past its last
-    // group), for the group sums of its rows.
+    // SwiGLU with ysum: h also goes to an LDS tile in natural column order
+    // (the ring stages, free once every wave is past its last group), for
+    // the group sums of its rows.
     constexpr int TS = BN + 8;                                     // bf16 per epilogue tile row
-    uint16_t* tile = reinterpret_cast<uint16_t*>(&st0);          // [64][TS] bf16
-    static_assert(64 * (BNW / 2 + 8) * 2 <= (int)sizeof(Stage), "epilogue tile");
+    uint16_t* tile = reinterpret_cast<uint16_t*>(&smem_all.ring[0]);   // [TBM][TS] bf16
+    static_assert(EPI != GEMM_SWIGLU || TBM * TS * 2 <= (int)sizeof(smem_all.ring), "epilogue tile");
     // whole-run vector stores: N % 4 == 0 and 8-byte aligned y and res
     // (16-byte aligned fp32 parts)
     const bool vec = N % 4 == 0 &&
-                     (S > 1 ? reinterpret_cast<uintptr_t>(p.part) % 16 == 0
+                     (S_K > 1 ? reinterpret_cast<uintptr_t>(p.part) % 16 == 0
                             : reinterpret_cast<uintptr_t>(p.y) % 8 == 0 &&
                                   (EPI != GEMM_RESIDUAL || reinterpret_cast<uintptr_t>(p.res) % 8 == 0));
     const float ascale = p.ascale != 0.0f ? p.ascale : 1.0f;
-    // The lane's four row scales, loaded together (one wait, not one per
-    // row tile).
-    float scv[4];
+    // The lane's row scales, loaded together (one wait, not one per row
+    // tile).
+    float scv[RI];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = m0 + i * 32 + col;
+    for (int i = 0; i < RI; ++i) {
+        const int row = m0 + (wr_ * RI + i) * 32 + col;
         scv[i] = (p.xscale && row < M ? p.xscale[row] : 1.0f) * ascale;
     }
-    // One-part residual epilogue: the residual runs of all four row tiles
+    // One-part residual epilogue: the residual runs of all row tiles
     // are loaded before the first is written (one wait, not one per run).
     // In place (res == y) every element is read and written by the same
     // lane, the read first.
-    const bool res_runs = EPI == GEMM_RESIDUAL && S == 1;
-    uint2 resv[4][4 * NJ];
+    const bool res_runs = EPI == GEMM_RESIDUAL && S_K == 1;
+    uint2 resv[RI][4 * NJ];
     const bool res_whole = vec && n0 + BN <= N;          // every run of the block: one 8-byte load
     auto load_res = [&](int i, uint2 (&rv)[4 * NJ]) {
-        const int row = m0 + i * 32 + col;
+        const int row = m0 + (wr_ * RI + i) * 32 + col;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int eg = 0; eg < 4; ++eg) {
-                const int cb = n0 + wave * (32 * NJ) + j * 32 + eg * 8 + h * 4;
+                const int cb = n0 + wc * (32 * NJ) + j * 32 + eg * 8 + h * 4;
                 uint2 t = make_uint2(0u, 0u);
                 if (row < M && cb < N) {
                     const uint16_t* r = p.res + (int64_t)row * N + cb;
@@ -466,9 +524,10 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
             // rows past M read row M - 1 (never stored): no branch between
             // the loads
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = m0 + i * 32 + col;
-                const uint16_t* r = p.res + (int64_t)(row < M ? row : M - 1) * N + n0 + wave * (32 * NJ) + h * 4;
+            for (int i = 0; i < RI; ++i) {
+                if (!mine(i)) continue;
+                const int row = m0 + (wr_ * RI + i) * 32 + col;
+                const uint16_t* r = p.res + (int64_t)(row < M ? row : M - 1) * N + n0 + wc * (32 * NJ) + h * 4;
 #pragma unroll
                 for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -477,15 +536,16 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) load_res(i, resv[i]);
+            for (int i = 0; i < RI; ++i)
+                if (mine(i)) load_res(i, resv[i]);
         }
     }
     // One wait for the row scales and residual runs, before the first branch
     // of the epilogue: past it the compiler's waits at branch joins would
     // count this tile's stores and drain them.
     wait_vmcnt<0>();
-    auto emit = [&](int i, int rbase) {
-        const int rl = i * 32 + col, row = m0 + rl;
+    auto emit = [&](int i) {
+        const int rl = (wr_ * RI + i) * 32 + col, row = m0 + rl;
         if (row >= M) return;
         const float sc = scv[i];
         const int64_t rowo = (int64_t)row * N;
@@ -498,13 +558,13 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
                 ga[e] = acc[i][0][e] * sc;
                 ua[e] = acc[i][1][e] * sc;
             }
-            swiglu_bf16_lut_batch<16>(ga, ua, hv, smem.lut);
+            swiglu_bf16_lut_batch<16>(ga, ua, hv, smem_all.lut);
         }
 #pragma unroll
         for (int j = 0; j < (NMAT == 2 ? 1 : NJ); ++j) {
 #pragma unroll
             for (int eg = 0; eg < 4; ++eg) {
-                const int cl = (NMAT == 2 ? wave * 32 : wave * (32 * NJ) + j * 32) + eg * 8 + h * 4;
+                const int cl = (NMAT == 2 ? wc * 32 : wc * (32 * NJ) + j * 32) + eg * 8 + h * 4;
                 const int cb = n0 + cl;                             // first column (position) of the run
                 if (cb >= N) continue;
                 const bool whole = vec && cb + 3 < N;
@@ -514,14 +574,15 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
                     for (int q = 0; q < 4; ++q) {
                         const uint32_t v = hv[eg * 4 + q];
                         o[q] = v;
-                        if (paired_out) tile[(rl - rbase) * TS + (cl & ~7) + perm8(h * 4 + q)] = (uint16_t)v;
+                        if (paired_out) tile[rl * TS + (cl & ~7) + perm8(h * 4 + q)] = (uint16_t)v;
                         if (f16_out) {
                             // exact for |h| within [2^-14, 65504] / yscale
                             const float hv = fminf(fmaxf(bf16_to_f32(v) * p.yscale, -65504.0f), 65504.0f);
                             o[q] = __builtin_bit_cast(uint16_t, (_Float16)hv);
                         }
                     }
-                    uint16_t* y = reinterpret_cast<uint16_t*>(p.y) + rowo + cb;
+                    uint16_t* y = reinterpret_cast<uint16_t*>(p.y) +
+                                  (f16_out ? ((int64_t)(cb >> 6) * M + row) * 64 + (cb & 63) : rowo + cb);
                     if (whole) {
                         *reinterpret_cast<uint2*>(y) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
                     } else {
@@ -534,7 +595,7 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
                 float v[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = acc[i][j][eg * 4 + q] * sc;
-                if (S > 1) {
+                if (S_K > 1) {
                     float* y = p.part + (int64_t)kpart * M * N + rowo + cb;
                     if (whole) {
                         *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
@@ -561,53 +622,83 @@ __global__ __launch_bounds__(kThreads, NJ == 1 ? 3 : 2) void q4_gemm16_kernel(Ge
             }
         }
     };
-    // ysum of group n0 / 64 + gi of rows rbase .. rbase + 63: thread t takes
-    // row t / 4, group (t / 2) % 2 and half t % 2 (32 values summed left to
-    // right), then the two halves are added (the order of mq4_gemm.hip's
-    // paired SwiGLU output)
-    auto group_sums = [&](int rbase) {
-        const int rl = tid >> 2, gi = (tid >> 1) & 1, hf = tid & 1;
-        float sum = 0.0f;
+    if (paired_out) __syncthreads();                               // every wave is done with the stages
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint4 v = *reinterpret_cast<const uint4*>(&tile[rl * TS + gi * 64 + hf * 32 + c * 8]);
-            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+    for (int i = 0; i < RI; ++i)
+        if (mine(i)) emit(i);
+    if constexpr (EPI == GEMM_SWIGLU) {
+        if (paired_out) {
+            // ysum of group n0 / 64 + gi of row rl: a task per row, group and
+            // half (32 values summed left to right), then the two halves are
+            // added (the order of mq4_gemm.hip's paired SwiGLU output)
+            constexpr int GI = BN / 64;
+            __syncthreads();
+            for (int t = tid; t < TBM * GI * 2; t += Sh::THREADS) {
+                const int rl = t / (2 * GI), gi = (t >> 1) % GI, hf = t & 1;
+                float sum = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                sum += bf16_to_f32(w4[q] & 0xffffu);
-                sum += bf16_to_f32(w4[q] >> 16);
+                for (int c = 0; c < 4; ++c) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(&tile[rl * TS + gi * 64 + hf * 32 + c * 8]);
+                    const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        sum += bf16_to_f32(w4[q] & 0xffffu);
+                        sum += bf16_to_f32(w4[q] >> 16);
+                    }
+                }
+                const float other = __shfl_xor(sum, 1);
+                if (hf == 0 && m0 + rl < M) p.ysum[(int64_t)((n0 >> 6) + gi) * M + m0 + rl] = sum + other;
             }
         }
-        const float other = __shfl_xor(sum, 1);
-        if (hf == 0 && m0 + rbase + rl < M)
-            p.ysum[(int64_t)((n0 >> 6) + gi) * M + m0 + rbase + rl] = sum + other;
-    };
-    if (paired_out) {
-        static_assert(kThreads == 4 * 64, "four threads per tile row");
-        __syncthreads();                                           // every wave is done with the stages
-        emit(0, 0);
-        emit(1, 0);
-        __syncthreads();
-        group_sums(0);
-        __syncthreads();                                           // the tile is read before rows 64-127
-        emit(2, 64);
-        emit(3, 64);
-        __syncthreads();
-        group_sums(64);
-    } else {
-        emit(0, 0);
-        emit(1, 0);
-        emit(2, 0);
-        emit(3, 0);
     }
+}
+
+// XCD-aware tile order (block b runs on XCD b % 8).  With many column blocks
+// (a multiple of 8) XCD x takes a fixed eighth of them for every row block,
+// so its weights stay in its own L2.  With few, that leaves one or two
+// columns per XCD and every XCD reads all of the activations (four times the
+// weights' bytes per tile): there XCD x takes a contiguous run of the row-major tile order instead.
+constexpr int kRowRunCols = 16;
+__device__ __forceinline__ void tile_of(int b, int T, int NB, int& nb, int& mb) {
+    const int x = b & 7, s = b >> 3;
+    if ((NB & 7) == 0 && NB > kRowRunCols) {
+        const int per = NB >> 3;
+        nb = (s % per) * 8 + x;
+        mb = s / per;
+    } else {
+        const int q = T >> 3, r = T & 7;
+        const int t = x * q + (x < r ? x : r) + s;
+        nb = t % NB;
+        mb = t / NB;
+    }
+}
+
+// WPE: waves per SIMD the registers are sized for.
+template <int EPI, int WR, int WC, int RI, int S, int KW, int WPE>
+__global__ __launch_bounds__(64 * WR * WC * KW, WPE) void q4_gemm16_kernel(Gemm16Args p) {
+    using Sh = Shape<WR, WC, RI, KW>;
+    constexpr int BN = Sh::BNW / (EPI == GEMM_SWIGLU ? 2 : 1);
+    __shared__ Smem<EPI, Sh::TBM, Sh::BNW, S, KW> smem;
+    static_assert(sizeof(smem) <= 160 * 1024, "LDS of a CU");
+    // K parts (GEMM_RESIDUAL): block b takes part b / tiles
+    const int S_K = EPI == GEMM_RESIDUAL && p.ksplit > 1 ? p.ksplit : 1;
+    int bt = blockIdx.x, kpart = 0;
+    if (S_K > 1) {
+        const int tiles = (int)gridDim.x / S_K;
+        kpart = bt / tiles;
+        bt -= kpart * tiles;
+    }
+    int nb, mb;
+    tile_of(bt, (int)gridDim.x / S_K, (p.N + BN - 1) / BN, nb, mb);
+    gemm16_tile<EPI, WR, WC, RI, S, KW>(p, smem, nb * BN, mb * Sh::TBM, kpart, S_K);
 }
 
 // ---------------------------------------------------------------------------
 // Activation pre-pass: one wave per row.  Pass 1 forms the row's sum of
 // squares (with the norm; the per-element formula of mq4_rms_norm) and the
 // largest |x (1 + w)| (|x| without the norm); pass 2 writes bf16(x r (1 + w))
-// (or x), scaled by 2^-e and converted to fp16, in the pair order, and
-// xscale[m] = 2^e.  e is the smallest such that the scaled row stays below
+// (or x), scaled by 2^-e and converted to fp16, in the pair order and by k
+// group ([group][row][64]), and xscale[m] = 2^e.  e is the smallest such that the scaled row stays below
 // 2^15 (0 for every normalized row whose values stay below 2^15).  With CAP >
 // 0 (K <= 512 CAP) a lane keeps its chunks of x and of the norm weight in
 // registers between the passes (all loads issued first), so the row is read
@@ -632,7 +723,7 @@ __global__ __launch_bounds__(256) void pair_rows16_kernel(const uint16_t* __rest
     const int CH = K / 8;
     const uint4* src = reinterpret_cast<const uint4*>(x + (int64_t)m * K);
     const uint4* nw4 = reinterpret_cast<const uint4*>(nw);
-    uint4* dst = reinterpret_cast<uint4*>(xp + (int64_t)m * K);
+    uint4* dst = reinterpret_cast<uint4*>(xp) + (int64_t)m * 8;       // chunk c: + (c / 8) M 8 + c % 8
     constexpr int NC = CAP > 0 ? CAP : 1;
     uint4 xc[NC], wc[NC];
     if (CAP > 0) {
@@ -688,7 +779,7 @@ __global__ __launch_bounds__(256) void pair_rows16_kernel(const uint16_t* __rest
                              (_Float16)(bf16_to_f32(pr[q] >> 16) * down)};
             o[q] = __builtin_bit_cast(uint32_t, hv);
         }
-        dst[c] = make_uint4(o[0], o[1], o[2], o[3]);
+        dst[(int64_t)(c >> 3) * M * 8 + (c & 7)] = make_uint4(o[0], o[1], o[2], o[3]);
     };
     if (CAP > 0) {
 #pragma unroll
@@ -703,22 +794,22 @@ __global__ __launch_bounds__(256) void pair_rows16_kernel(const uint16_t* __rest
 
 // y = bf16(res + round_bf16(part[0] + part[1] + ... + part[S - 1])), the
 // parts added in order: 4 elements per thread (MN % 4 == 0, 16-byte aligned
-// parts, 8-byte aligned res and y), S <= 4.
+// parts, 8-byte aligned res and y), S <= 6.
 __global__ __launch_bounds__(256) void kpart_residual_kernel(const float* __restrict__ part, int S, int64_t MN,
                                                              const uint16_t* __restrict__ res,
                                                              uint16_t* __restrict__ y) {
 #pragma clang fp contract(off)
     const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (e >= MN) return;
-    // every load issued before the first add (S <= 4 parts)
-    float4 v[4];
+    // every load issued before the first add (S <= 6 parts)
+    float4 v[6];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < 6; ++k)
         if (k < S) v[k] = *reinterpret_cast<const float4*>(part + (int64_t)k * MN + e);
     const uint2 r = *reinterpret_cast<const uint2*>(res + e);
     float4 sum = v[0];
 #pragma unroll
-    for (int k = 1; k < 4; ++k) {
+    for (int k = 1; k < 6; ++k) {
         if (k < S) {
             sum.x += v[k].x;
             sum.y += v[k].y;
@@ -757,49 +848,99 @@ int launch_pair_rows16(const uint16_t* x, int M, int K, const uint16_t* norm_w, 
     return 0;
 }
 
+namespace g16 {
+
+// The tile of a product: rows x weight columns (gate/up: half of them each).
+//   T64x128:  two teams of 2 waves (64 x 64 each) on halves of K, 4 stages
+//   T128x128: 4 waves of 64 x 64, 4 stages
+//   T128x256: 4 waves of 128 x 64, 2 stages, two blocks per CU
+//   T256x256: 8 waves of 128 x 64, 2 stages
+// Few rows leave CUs idle and each block serial: the smallest tile whose
+// blocks are all resident at one per CU.  Many rows: the fewest VALU per
+// MFMA, which is 128 rows per wave.  Measured, us per kernel (gate/up 2 x
+// 6144 x 2048, and down 2048 x 6144 in the parts of gemm16_parts):
+//   M      gate/up, 64x128 / 128x128 / 128x256    down, the same / 256x256
+//   40     13.5 / 20.4 / 28.0                     10.4 / 12.1 (6 parts)
+//   203    26.8 / 20.7 / 32.2                     16.6 (3) / 15.2 (6) / 79 (1)
+//   400    38.6 / 40.1 / 33.5                     21.7 (2) / 20.2 (4)
+//   1960   152 / 124 / 102                        76 / 62 / 86 / 119 (1 part)
+//   2560   -   / -   / 123                        104 (128x128) / 90 / 125
+//   6000   -   / -   / 275 (256x256: 294)         174 (128x128) / 160 / 150
+// (every shape in one stage less and the dequantization waiting for its
+// operands, 128 x 256 and 128 x 128 tiles: 33 / 37 / 36 / 107 / 141 / 310 us
+// gate/up and 17 / 19 / 21 / 73 / 105 / 189 us down.)
+enum Tile { T64x128, T128x128, T128x256, T256x256 };
+Tile tile_for(int64_t M, int64_t N, int64_t K, int epi) {
+    const int64_t cols = epi == GEMM_SWIGLU ? 2 * N : N, cus = num_cus();
+    auto blocks = [&](int r, int c) { return ((M + r - 1) / r) * ((cols + c - 1) / c); };
+    const bool teams = (K / 64) % 16 == 0;             // eight-group blocks in each half of K
+    if (teams && (epi == GEMM_SWIGLU ? blocks(64, 128) <= cus : M <= 128)) return T64x128;
+    if (blocks(128, 128) <= cus) return T128x128;
+    if (epi == GEMM_SWIGLU || blocks(128, 256) <= cus) return T128x256;
+    return T256x256;
+}
+
+}  // namespace g16
+
+// The most K parts (whole eight-group blocks per part and team) whose blocks
+// stay within one per CU.
+int gemm16_parts(int64_t M, int64_t N, int64_t K) {
+    const g16::Tile t = g16::tile_for(M, N, K, GEMM_RESIDUAL);
+    const int64_t r = t == g16::T64x128 ? 64 : t == g16::T256x256 ? 256 : 128;
+    const int64_t c = t == g16::T64x128 || t == g16::T128x128 ? 128 : 256;
+    const int64_t blocks = ((M + r - 1) / r) * ((N + c - 1) / c), teams = t == g16::T64x128 ? 2 : 1;
+    int S = 1;
+    for (int s : {2, 3, 4, 6})
+        if ((K / 512) % (s * teams) == 0 && blocks * s <= (int64_t)num_cus()) S = s;
+    return S;
+}
+
 int launch_q4_gemm16(const Gemm16Args& a, int epi, hipStream_t st) {
     // 32-bit byte offsets in the kernel; whole blocks of 8 groups (K % 512,
     // the scale/bias DMA) with scale/bias rows 16-byte aligned
     const bool fits32 = (int64_t)a.M * a.K * 2 <= 0xFFFFFFFFLL && (int64_t)a.N * a.K / 2 <= 0xFFFFFFFFLL;
     auto a16 = [](const QMat& q) { return reinterpret_cast<uintptr_t>(q.s) % 16 == 0 && reinterpret_cast<uintptr_t>(q.b) % 16 == 0; };
+    if (epi != GEMM_SWIGLU && epi != GEMM_RESIDUAL) return -1;
     if (!fits32 || a.K % 512 != 0 || a.M < 1 || a.N < 1 || !a16(a.A) || (epi == GEMM_SWIGLU && !a16(a.B))) return -1;
     if (a.ysum && (epi != GEMM_SWIGLU || a.yscale != 0.0f || a.N % 128 != 0)) return -1;
     if (a.yscale != 0.0f && (epi != GEMM_SWIGLU || a.N % 8 != 0)) return -1;
     if (epi == GEMM_SWIGLU && (!a.silu_lut || !aligned(a.silu_lut, 16))) return -1;
-    // K parts: GEMM_RESIDUAL only, at most 4, whole 8-group scale slots per
+    // K parts: GEMM_RESIDUAL only, at most 6, whole 8-group scale slots per
     // part, fp32 parts [ksplit][M][N] (16-byte aligned, N % 4 == 0) combined
     // by a second kernel
     const int S = a.ksplit > 1 ? a.ksplit : 1;
-    if (S > 1 && (epi != GEMM_RESIDUAL || S > 4 || (a.K / 64) % (8 * S) != 0 || !a.part ||
+    if (S > 1 && (epi != GEMM_RESIDUAL || S > 6 || (a.K / 64) % (8 * S) != 0 || !a.part ||
                   reinterpret_cast<uintptr_t>(a.part) % 16 != 0 || a.N % 4 != 0 || !aligned(a.res, 8) ||
                   !aligned(a.y, 8)))
         return -1;
-    // 128-column tiles (three blocks per CU) for the residual product when
-    // asked for, else 256
-    const bool narrow = epi == GEMM_RESIDUAL && a.narrow;
-    const int BN = epi == GEMM_SWIGLU ? g16::Cols<2>::BNW / 2 : narrow ? g16::Cols<1>::BNW : g16::Cols<2>::BNW;
-    const unsigned blocks = (unsigned)(((a.N + BN - 1) / BN) * ((a.M + g16::TBM - 1) / g16::TBM) * S);
-    switch (epi) {
-        case GEMM_RESIDUAL: {
-            if (narrow)
-                hipLaunchKernelGGL((g16::q4_gemm16_kernel<GEMM_RESIDUAL, 1>), dim3(blocks), dim3(g16::kThreads), 0, st,
-                                   a);
-            else
-                hipLaunchKernelGGL((g16::q4_gemm16_kernel<GEMM_RESIDUAL, 2>), dim3(blocks), dim3(g16::kThreads), 0, st,
-                                   a);
-            if (S > 1) {
-                const int64_t MN = (int64_t)a.M * a.N;
-                hipLaunchKernelGGL(g16::kpart_residual_kernel, dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0,
-                                   st, a.part, S, MN, a.res, reinterpret_cast<uint16_t*>(a.y));
-            }
-            return 0;
+    const unsigned cols = (unsigned)(epi == GEMM_SWIGLU ? 2 * a.N : a.N);
+    auto go = [&](auto kern, int threads, int tbm, int bnw) {
+        const unsigned blocks = (cols + bnw - 1) / bnw * (unsigned)((a.M + tbm - 1) / tbm) * S;
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), 0, st, a);
+    };
+    using namespace g16;
+    const Tile t = tile_for(a.M, a.N, a.K, epi);
+    if (t == T64x128 && (a.K / 64) % (16 * S) != 0) return -1;
+    if (epi == GEMM_SWIGLU) {
+        switch (t) {
+            case T64x128: go(q4_gemm16_kernel<GEMM_SWIGLU, 1, 2, 2, 4, 2, 1>, 256, 64, 128); break;
+            case T128x128: go(q4_gemm16_kernel<GEMM_SWIGLU, 2, 2, 2, 4, 1, 1>, 256, 128, 128); break;
+            default: go(q4_gemm16_kernel<GEMM_SWIGLU, 1, 4, 4, 2, 1, 2>, 256, 128, 256); break;
         }
-        case GEMM_SWIGLU:
-            hipLaunchKernelGGL((g16::q4_gemm16_kernel<GEMM_SWIGLU, 2>), dim3(blocks), dim3(g16::kThreads), 0, st, a);
-            return 0;
-        default:
-            return -1;
+        return 0;
     }
+    switch (t) {
+        case T64x128: go(q4_gemm16_kernel<GEMM_RESIDUAL, 1, 2, 2, 4, 2, 1>, 256, 64, 128); break;
+        case T128x128: go(q4_gemm16_kernel<GEMM_RESIDUAL, 2, 2, 2, 4, 1, 1>, 256, 128, 128); break;
+        case T128x256: go(q4_gemm16_kernel<GEMM_RESIDUAL, 1, 4, 4, 2, 1, 2>, 256, 128, 256); break;
+        case T256x256: go(q4_gemm16_kernel<GEMM_RESIDUAL, 2, 4, 4, 2, 1, 2>, 512, 256, 256); break;
+    }
+    if (S > 1) {
+        const int64_t MN = (int64_t)a.M * a.N;
+        hipLaunchKernelGGL(g16::kpart_residual_kernel, dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, st,
+                           a.part, S, MN, a.res, reinterpret_cast<uint16_t*>(a.y));
+    }
+    return 0;
 }
 
 }  // namespace mq4

@@ -756,7 +756,7 @@ namespace mq4 {
 // part [2, M, K] fp32 holds the two K parts of the split down product.  On
 // the fp16-weight path the down product in S > 1 K parts puts them in
 // kpart [S, M, K] fp32, and silu holds the SwiGLU epilogue's table of the
-// rounded SiLU (SILU_LUT_N bf16, written by the pre-pass).  Sections 256-byte
+// rounded sigmoid (SILU_LUT_N bf16, written by the pre-pass).  Sections 256-byte
 // aligned.
 struct MlpWs {
     uint16_t* h = nullptr;
@@ -770,34 +770,9 @@ struct MlpWs {
     size_t bytes = 0;
 };
 
-// Tiles and K parts of the fp16-weight down product ([M, N] . [K, N]^T,
-// N / 64 groups) on the one-call path: 128 x 128 tiles (three blocks per CU)
-// while there are at most two of them per CU, else 128 x 256; and the most
-// of 1, 2 and 4 parts (whole 8-group scale slots per part) whose tiles times
-// parts stay within one block per CU.  Measured on the 2048 x 6144 down
-// product with its part combine, us for 1 / 2 / 4 parts, 128 x 256 tiles then
-// 128 x 128:
-//   M = 200:  84.4 / 48.6 / 31.0,    55.2 / 33.2 / 22.5
-//   M = 1024: 91.7 / 54.8 / 45.6,    61.0 / 42.7 / 45.0
-//   M = 2048: 99.1 / 71.2 / 79.1,    69.8 / 71.2 / 80.4
-//   M = 3072: 108.0 / 105.0 / 113.4, 101.4 / 101.6 / 114.8
-//   M = 4096: 119.5 / 126.2 / 146.4, 118.0 / 133.3 / 150.9
-//   M = 8192: 212.5 / 250.5 / 315.0, 230.4 / 268.6 / 332.4
-// Either tile width gives the same bits.  0 parts: N / 64 not a multiple of
-// 8 (no fp16 down product).
-static bool mlp_down_narrow(int64_t M, int64_t K) {
-    return ((M + 127) / 128) * ((K + 127) / 128) <= 2 * (int64_t)num_cus();
-}
-static int mlp_down_parts(int64_t M, int64_t K, int64_t N) {
-    const int64_t G = N / 64;
-    if (N % 64 != 0 || G % 8 != 0) return 0;
-    const int64_t BN = mlp_down_narrow(M, K) ? 128 : 256;
-    const int64_t tiles = ((M + 127) / 128) * ((K + BN - 1) / BN);
-    int S = 1;
-    for (int s : {2, 4})
-        if ((G / 8) % s == 0 && tiles * s <= (int64_t)num_cus()) S = s;
-    return S;
-}
+// K parts of the fp16-weight down product ([M, N] . [K, N]^T); 0: N / 64 not
+// a multiple of 8 (no fp16 down product).
+static int mlp_down_parts(int64_t M, int64_t K, int64_t N) { return N % 512 != 0 ? 0 : gemm16_parts(M, K, N); }
 
 static MlpWs mlp_ws_layout(void* base, int64_t M, int64_t K, int64_t N) {
     MlpWs w;
@@ -840,7 +815,7 @@ static bool mlp_paired_ok(int64_t M, int64_t K, int64_t N, const QMat& g, const 
 // only; to kGemmMinM - 1: h and two fp32 K parts; from kGemmMinM: h, the
 // paired operands and the down product's K parts), except where the K-part
 // count drops, so the size is the largest over the regimes' top row counts
-// and the row counts just below a drop (multiples of 128), up to M.
+// and the row counts just below a drop (multiples of 64), up to M.
 extern "C" size_t mq4_mlp_workspace_size(int64_t M, int64_t K, int64_t N) {
     if (M <= 0 || K <= 0 || N <= 0) return 0;
     size_t need = mlp_ws_layout(nullptr, M, K, N).bytes;
@@ -851,8 +826,11 @@ extern "C" size_t mq4_mlp_workspace_size(int64_t M, int64_t K, int64_t N) {
     };
     at(kMfmaMinM - 1);
     at(kGemmMinM - 1);
-    for (int64_t m = 128; m < M; m += 128)
-        if (mlp_down_parts(m, K, N) > mlp_down_parts(m + 1, K, N)) at(m);
+    for (int64_t m = 64; m < M; m += 64) {
+        const int parts = mlp_down_parts(m, K, N);
+        if (m > 128 && parts <= 1) break;              // one part from here on
+        if (parts > mlp_down_parts(m + 1, K, N)) at(m);
+    }
     return need;
 }
 
@@ -881,9 +859,9 @@ extern "C" int mq4_mlp_residual(const uint16_t* x, int64_t M, int64_t K, const u
         // SwiGLU on an fp16 copy of the normalized x (its per-row
         // power-of-two scales in the xs area), and the down product on h
         // written as fp16 / 256 in the operand order (exact for |h| in
-        // [2^-6, 1.6e7]), with the tiles and K parts of mlp_down_parts (2048
-        // x 6144 down at M = 2048: 70 us, against 102 us on the
-        // exact-operand GEMM with paired bf16 h).  With the down product's scale or bias rows
+        // [2^-6, 1.6e7]), in the K parts of mlp_down_parts (2048 x 6144 down
+        // at M = 1960: 62 us, against 102 us on the exact-operand GEMM with
+        // paired bf16 h).  With the down product's scale or bias rows
         // not 16-byte aligned, gate/up writes h paired in bf16 with its group
         // sums for the exact-operand GEMM's down product.
         auto a16 = [](const QMat& q) { return aligned(q.s, 16) && aligned(q.b, 16); };
@@ -896,12 +874,12 @@ extern "C" int mq4_mlp_residual(const uint16_t* x, int64_t M, int64_t K, const u
             if (launch_pair_rows16(x, (int)M, (int)K, norm_weight, eps, w.xp, w.xs, w.silu, st))
                 return fail(MQ4_ERR_UNSUPPORTED, "%s: unsupported shape", what);
             Gemm16Args gu{w.xp, w.xs, (int)M, (int)N, (int)K, G, U, w.hp, nullptr, down16 ? nullptr : w.hs, 0.0f,
-                          down16 ? 1.0f / 256.0f : 0.0f, 0, nullptr, 0, w.silu};
+                          down16 ? 1.0f / 256.0f : 0.0f, 0, nullptr, w.silu};
             if (launch_q4_gemm16(gu, GEMM_SWIGLU, st))
                 return fail(MQ4_ERR_UNSUPPORTED, "%s: unsupported shape", what);
             if (down16) {
                 Gemm16Args dn{w.hp, nullptr, (int)M, (int)K, (int)N, D, QMat{nullptr, nullptr, nullptr}, y, x,
-                              nullptr, 256.0f, 0.0f, parts, w.kpart, mlp_down_narrow(M, K) ? 1 : 0};
+                              nullptr, 256.0f, 0.0f, parts, w.kpart, nullptr};
                 if (launch_q4_gemm16(dn, GEMM_RESIDUAL, st))
                     return fail(MQ4_ERR_UNSUPPORTED, "%s: unsupported shape", what);
                 return launch_status(what);

@@ -430,3 +430,35 @@ def test_mlp_residual_split_graph_replay(mq4, O, dev, M):
         assert np.array_equal(to_host_u16(y), want), f"replay {r}"
         mq4.qmatmul(x, w.gate_proj)                        # eager work between replays
         torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(33, 2048, 6144), (64, 2048, 6144), (65, 2048, 6144), (128, 2048, 6144),
+                                   (129, 2048, 6144), (192, 2048, 6144), (256, 2048, 6144), (257, 2048, 6144),
+                                   (385, 2048, 6144), (513, 2048, 6144), (2049, 2048, 6144), (4097, 2048, 6144),
+                                   (33, 1024, 3072), (320, 1024, 3072), (321, 1024, 3072), (129, 512, 512),
+                                   (385, 1024, 1536)])
+def test_mlp_residual_tile_edges(mq4, O, dev, M, K, N):
+    """The one-call MLP at the row counts where its tiles and K parts change
+    (64 x 128 tiles on two K teams up to 128 rows, 128 x 128, 128 x 256 and
+    256 x 256 beyond; 6, 4, 3, 2 and 1 down parts) and one past them, against
+    the separate entries, which run the exact-operand kernels: the bounds of
+    test_mlp_residual_one_call (>= 95% of the bits, the rounding flips of the
+    fp16 weights and of the K parts' sums; rms of the difference <= 1e-2)."""
+    import torch
+    print(f"mlp_residual tile edges M={M} K={K} N={N}", flush=True)
+    ws = [make(mq4, O, *((N, K) if p < 2 else (K, N)), 1700 + p, dev) for p in range(3)]
+    w = mq4.MLPWeights(*[mq4.QuantizedTensor(*d) for d, _ in ws])
+    x = mq4.fill_normal_bf16((M, K), mq4.STREAM_PREFILL + 7, 0.0, 1.0, device=dev)
+    nw = mq4.fill_normal_bf16((K,), mq4.stream_id_layer_norm(5), 0.1, 0.02, device=dev)
+    guard = torch.full((M + 1, K), 7.0, dtype=torch.bfloat16, device=dev)
+    y = mq4.mlp_residual(x, w, nw, 1e-6, out=guard[:M])
+    h = mq4.mlp_gate_up_silu(x, w.gate_proj, w.up_proj, norm_weight=nw, eps=1e-6)
+    ys = mq4.qmatmul_residual(h, w.down_proj, x)
+    torch.cuda.synchronize()
+    assert bool((guard[M] == 7.0).all()), "a row past M was written"
+    same = float((y.view(torch.int16) == ys.view(torch.int16)).float().mean())
+    d, m = y.double() - ys.double(), ys.double() - x.double()
+    rel = float(d.norm() / m.norm())
+    print(f"identical {same:.5f}, rms(diff)/rms(mlp) {rel:.2e}")
+    assert same >= 0.95 and rel <= TOL
