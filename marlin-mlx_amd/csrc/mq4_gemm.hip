@@ -44,12 +44,17 @@
 //    XCDs, each XCD takes a fixed eighth of the column blocks for every row
 //    block, so its weights stay in its own L2 across the row blocks.
 //  * LDS rows are padded to 72 bf16 (144 bytes) against bank conflicts.
+// This first kernel (q4_gemm_kernel) serves the fused norm and the odd group
+// counts and alignments; the others stage every operand by LDS DMA: the ring
+// kernel (namespace ring) whole eight-group blocks of K, q4_gemm_dma_kernel
+// the rest and the pre-paired operands.
 #include <type_traits>
 
 #include "mq4_device.h"
 #include "mq4_gemm.h"
 #include "mq4_gemv.h"
 #include "mq4_host.h"
+#include "mq4_stage.h"
 
 namespace mq4 {
 
@@ -685,6 +690,446 @@ void launch_dma_auto(const GemmArgs& a, hipStream_t st) {
 
 }  // namespace dma
 
+// ---------------------------------------------------------------------------
+// The same product for whole eight-group blocks of K (K % 512 == 0, K >= 1024) and
+// 16-byte aligned scale and bias rows, on the ring and schedule of the
+// fp16-weight GEMM (mq4_gemm16.hip): a block of KW teams of WR x WC waves,
+// each wave 64 rows x 64 weight columns, the teams on their own parts of K.
+//
+// A wave issues about 200 VALU per k group (64 folds, 56 nibble unpacks, 64
+// permutes and group sums of the activations) against 16 MFMAs of 14 ns, so
+// the VALU bounds it (2.0 ns each with two waves per SIMD, 2.4 with one): the
+// loop holds nothing else.  Eight groups are unrolled, so that every LDS
+// address is a constant; scales and biases are read once per eight groups;
+// the next MFMA step's operands are read and formed during the current one;
+// the group's fold waits until the next group's first MFMA step, one tile at
+// a time ahead of the MFMA that overwrites it.  So an MFMA result is read no
+// sooner than 45 instructions after its issue (counted in the built loop),
+// well past the wait states that mfma_result_pad stands for.
+namespace ring {
+
+constexpr int RI = 2, NJ = 2;             // 32 x 32 MFMA tiles of a wave: rows, weight columns
+
+template <int WR, int WC, int KW>
+struct Shape {
+    static constexpr int NW = WR * WC, THREADS = 64 * NW * KW;
+    static constexpr int TBM = 32 * RI * WR;            // rows per block
+    static constexpr int BNW = 32 * NJ * WC;            // weight columns per block
+    static constexpr int A_I = TBM / 8 / NW;            // activation DMA instructions per wave and group
+    static constexpr int B_I = BNW / 32 / NW;           // weight DMA instructions per wave and group
+    static constexpr int SB_I = 2 * BNW / 64 / NW;      // scale/bias DMA instructions per wave and 8 groups
+    static_assert(A_I * 8 * NW == TBM && B_I * 32 * NW == BNW && SB_I * 64 * NW == 2 * BNW,
+                  "every wave issues the same DMA");
+};
+
+// One k group: activations [row][chunk ^ ((row >> 1) & 7)] (bf16, natural
+// order) and packed weights [32-column block][k-half][column].
+template <int TBM, int BNW>
+struct Stage {
+    uint4 a[TBM * 8];
+    uint4 b[2 * BNW];
+};
+// A team's S stages, and the scales and biases of 8 groups, [scales |
+// biases][weight column], 16 bytes each, in two slots.
+template <int TBM, int BNW, int S>
+struct Ring {
+    Stage<TBM, BNW> st[S];
+    uint4 sb[2][2][BNW];
+};
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <int EPI, int WR, int WC, int S, int KW>
+__global__ __launch_bounds__(64 * WR * WC * KW, 2) void q4_gemm_ring_kernel(GemmArgs p) {
+#pragma clang fp contract(off)
+    using Sh = Shape<WR, WC, KW>;
+    constexpr int NMAT = EPI == GEMM_SWIGLU ? 2 : 1;
+    constexpr int TBM = Sh::TBM, BNW = Sh::BNW, A_I = Sh::A_I, B_I = Sh::B_I, SB_I = Sh::SB_I;
+    constexpr int BN = BNW / NMAT;                       // output columns per block
+    constexpr int D_I = A_I + B_I;                       // DMA instructions per wave and stage
+    static_assert((S == 2 || S == 4) && D_I * (S - 1) < 64, "ring depth");
+    __shared__ Ring<TBM, BNW, S> rings[KW];
+    static_assert(sizeof(rings) <= 160 * 1024, "LDS of a CU");
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int bwave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int team = bwave / Sh::NW, wave = bwave % Sh::NW;
+    const int wm = wave / WC, wn = wave % WC;
+    const int h = lane >> 5, col = lane & 31;
+    const int M = p.M, N = p.N, K = p.K, G = K / 64;
+    const int GL = G / KW, g0 = team * GL;               // this team's groups
+    auto& smem = rings[team];
+
+    // block -> tile: XCD x (block b runs on XCD b % 8) takes a contiguous run
+    // of the row-major tile order, or with many column blocks a fixed eighth
+    // of them for every row block (its weights stay in its own L2)
+    const int NB = (N + BN - 1) / BN;
+    int nb, mb;
+    {
+        const int b = blockIdx.x, x = b & 7, s = b >> 3, T = gridDim.x;
+        if ((NB & 7) == 0 && NB > 16) {
+            const int per = NB >> 3;
+            nb = (s % per) * 8 + x;
+            mb = s / per;
+        } else {
+            const int q = T >> 3, r = T & 7, t = x * q + (x < r ? x : r) + s;
+            nb = t % NB;
+            mb = t / NB;
+        }
+    }
+    const int n0 = nb * BN, m0 = mb * TBM;
+
+    // ---- DMA sources: wave-uniform pointers, moved along K one group per
+    // step, plus 32-bit lane byte offsets (rows past the end repeat the last) ----
+    const char* xp = reinterpret_cast<const char*>(p.x) + (int64_t)g0 * 128;
+    uint32_t aoff[A_I];
+#pragma unroll
+    for (int t = 0; t < A_I; ++t) {
+        const int slot = (wave * A_I + t) * 64 + lane;
+        const int r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
+        const int row = (m0 + r) < M ? (m0 + r) : (M - 1);
+        aoff[t] = (uint32_t)(((int64_t)row * K + c * 8) * 2);
+    }
+    auto wrow_of = [&](int r) -> int {
+        const int n = NMAT == 2 ? n0 + (r % (BNW / 2)) : n0 + r;
+        return n < N ? n : N - 1;
+    };
+    auto mat_of = [&](int r) -> const QMat& { return (NMAT == 2 && r >= BNW / 2) ? p.B : p.A; };
+    const char* bp[B_I];
+    uint32_t boff[B_I];
+#pragma unroll
+    for (int t = 0; t < B_I; ++t) {
+        const int r0 = (wave * B_I + t) * 32;            // 32 weight columns, k-half lane / 32
+        bp[t] = reinterpret_cast<const char*>(mat_of(r0).wq) + (int64_t)g0 * 32;
+        boff[t] = (uint32_t)((int64_t)wrow_of(r0 + (lane & 31)) * (K / 2) + (lane >> 5) * 16);
+    }
+    // scales and biases, 16 bytes (8 groups) of one weight column per lane;
+    // with 64 weight columns one instruction covers gate and up columns
+    const char* sbp[SB_I];
+    uint32_t sboff[SB_I];
+    static_assert(NMAT == 1 || BNW >= 128, "one matrix per scale/bias DMA instruction");
+#pragma unroll
+    for (int t = 0; t < SB_I; ++t) {
+        const int u0 = (wave * SB_I + t) * 64, sel = u0 / BNW, r0 = u0 % BNW;
+        sbp[t] = reinterpret_cast<const char*>(sel ? mat_of(r0).b : mat_of(r0).s) + (int64_t)(g0 / 8) * 16;
+        sboff[t] = (uint32_t)((int64_t)wrow_of(r0 + lane) * G * 2);
+    }
+    const uint32_t a_lds = stage::lds_addr(&smem.st[0].a[0]) + (uint32_t)(wave * A_I * 1024);
+    const uint32_t b_lds = stage::lds_addr(&smem.st[0].b[0]) + (uint32_t)(wave * B_I * 1024);
+    const uint32_t sb_lds = stage::lds_addr(&smem.sb[0][0][0]) + (uint32_t)(wave * SB_I * 1024);
+    constexpr uint32_t STG = sizeof(smem.st[0]), SBS = sizeof(smem.sb[0]);
+    auto issue = [&](int slot, int step) {               // then the pointers move on by `step` groups
+#pragma unroll
+        for (int t = 0; t < A_I; ++t) stage::dma16_m0(xp, aoff[t], a_lds + slot * STG + t * 1024);
+#pragma unroll
+        for (int t = 0; t < B_I; ++t) stage::dma16_m0(bp[t], boff[t], b_lds + slot * STG + t * 1024);
+        xp += step * 128;
+#pragma unroll
+        for (int t = 0; t < B_I; ++t) bp[t] += step * 32;
+    };
+    auto issue_sb = [&](uint32_t slot, int step) {
+#pragma unroll
+        for (int t = 0; t < SB_I; ++t) {
+            stage::dma16_m0(sbp[t], sboff[t], sb_lds + slot * SBS + t * 1024);
+            sbp[t] += step * 16;
+        }
+    };
+
+    // ---- operands: LDS slots of this lane (row tile i: + 256 i) ----
+    int wr[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) wr[j] = NMAT == 2 ? j * (BNW / 2) + wn * 32 + col : wn * (32 * NJ) + j * 32 + col;
+    uint32_t arow[4], brow[NJ];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) arow[ks] = (uint32_t)((wm * RI * 32 + col) * 8 + ((4 * h + ks) ^ ((col >> 1) & 7)));
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) brow[j] = (uint32_t)((wr[j] >> 5) * 64 + h * 32 + (wr[j] & 31));
+    const uint32_t ONES = 0x3f803f80u;                   // bf16 pair (1, 1)
+    uint32_t nib_mask, nib_exp;
+    asm("s_mov_b32 %0, 0x000f000f" : "=s"(nib_mask));
+    asm("v_mov_b32 %0, 0x43004300" : "=v"(nib_exp));
+
+    f32x16_t acc[RI][NJ], D[RI][NJ];
+#pragma unroll
+    for (int i = 0; i < RI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = D[i][j][e] = 0.0f;
+    const f32x16_t zero = acc[0][0];
+    uint4 bw[NJ], sv[NJ], bv[NJ];                        // a group's words; eight groups' scales and biases
+    float s[NJ], c[NJ], xs[RI];                          // the group being read: scale, bias - 128 scale, sums
+    float sf[NJ];                                        // the group to fold
+    float xe[RI], ce[NJ];                                // the even group of a pair
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) sf[j] = ce[j] = 0.0f;
+    auto read_w = [&](int slot) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) bw[j] = smem.st[slot].b[brow[j]];
+    };
+    auto read_sb = [&](uint32_t slot) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            sv[j] = smem.sb[slot][0][wr[j]];
+            bv[j] = smem.sb[slot][1][wr[j]];
+        }
+    };
+    auto group_sb = [&](int u) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t sw = word_of(sv[j], u >> 1), bwd = word_of(bv[j], u >> 1);
+            s[j] = __uint_as_float(u & 1 ? sw & 0xffff0000u : sw << 16);
+            c[j] = __uint_as_float(u & 1 ? bwd & 0xffff0000u : bwd << 16) - 128.0f * s[j];   // affine_c
+        }
+    };
+    auto read_a = [&](int slot, int ks, uint4 (&r)[RI]) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i) r[i] = smem.st[slot].a[arow[ks] + 256 * i];
+    };
+    // one MFMA step's operands: activations in the nibble-pair order (x0,
+    // x4), (x1, x5), (x2, x6), (x3, x7) with their sum, exact 128 + q
+    auto form = [&](int ks, const uint4 (&r)[RI], bf16x8_t (&a)[RI], bf16x8_t (&b)[NJ]) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            const uint4 v = r[i];
+            xs[i] = dot2_bf16(v.w, ONES, dot2_bf16(v.z, ONES, dot2_bf16(v.y, ONES, dot2_bf16(v.x, ONES, xs[i]))));
+            a[i] = __builtin_bit_cast(
+                bf16x8_t, make_uint4(__builtin_amdgcn_perm(v.z, v.x, dma::kPermLo), __builtin_amdgcn_perm(v.z, v.x, dma::kPermHi),
+                                     __builtin_amdgcn_perm(v.w, v.y, dma::kPermLo), __builtin_amdgcn_perm(v.w, v.y, dma::kPermHi)));
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) b[j] = weight_operand_k(word_of(bw[j], ks), nib_mask, nib_exp);
+    };
+    auto mfmas = [&](const bf16x8_t (&a)[RI], const bf16x8_t (&b)[NJ]) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], D[i][j], 0, 0, 0);
+    };
+    auto fold = [&](int i, int j) {                      // acc += s D of the last group
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = __builtin_fmaf(sf[j], D[i][j][e], acc[i][j][e]);
+    };
+    // acc += (b - 128 s) X of two groups on the fp32 MFMA: lanes 0-31 carry
+    // the even one, lanes 32-63 the odd one
+    auto offsets = [&](const float (&xo)[RI], const float (&co)[NJ]) {
+#pragma unroll
+        for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(h ? xo[i] : xe[i], h ? co[j] : ce[j], acc[i][j], 0, 0, 0);
+    };
+
+    const int nblk = GL / 8;
+    issue_sb(0, nblk > 1 ? 1 : 0);
+#pragma unroll
+    for (int t = 0; t < S; ++t) issue(t, 1);             // GL >= 8 > S
+    wait_vmcnt<D_I * (S - 1)>();
+    lds_barrier();
+    uint4 r0[RI], r1[RI];
+    bf16x8_t a0[RI], a1[RI], b0[NJ], b1[NJ];
+    read_w(0);
+    read_sb(0);
+    read_a(0, 0, r0);
+    read_a(0, 1, r1);
+#pragma unroll
+    for (int i = 0; i < RI; ++i) xs[i] = 0.0f;
+    group_sb(0);
+    form(0, r0, a0, b0);
+
+    for (int t8 = 0; t8 < nblk; ++t8) {
+        const int inc = t8 + 1 < nblk ? 1 : 0, sb_inc = t8 + 2 < nblk ? 1 : 0;
+        const uint32_t nsb = (uint32_t)(t8 + 1) & 1;
+        auto step = [&](auto uc) {
+            constexpr int u = decltype(uc)::value, cs = u % S, ns = (u + 1) % S;
+            // MFMA step 0: the last group's fold, a tile ahead of the MFMA that replaces it
+            read_a(cs, 2, r0);
+#pragma unroll
+            for (int i = 0; i < RI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    fold(i, j);
+                    D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[i], b0[j], zero, 0, 0, 0);
+                }
+            form(1, r1, a1, b1);
+            __builtin_amdgcn_sched_barrier(0);
+            read_a(cs, 3, r1);
+            mfmas(a1, b1);
+            form(2, r0, a0, b0);
+            __builtin_amdgcn_sched_barrier(0);
+            mfmas(a0, b0);
+            form(3, r1, a1, b1);
+            float X[RI], co[NJ];
+#pragma unroll
+            for (int i = 0; i < RI; ++i) {
+                float lo, hi;
+                swap_halves<32>(xs[i], xs[i], lo, hi);
+                X[i] = lo + hi;
+                xs[i] = 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                sf[j] = s[j];
+                co[j] = c[j];
+            }
+            if constexpr ((u & 1) == 0) {
+#pragma unroll
+                for (int i = 0; i < RI; ++i) xe[i] = X[i];
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) ce[j] = co[j];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            wait_vmcnt<D_I * (S - 2)>();
+            lds_barrier();
+            read_w(ns);
+            if constexpr (u == 7) read_sb(nsb);          // past the end: stale bytes, not used
+            read_a(ns, 0, r0);
+            read_a(ns, 1, r1);
+            mfmas(a1, b1);
+            issue(cs, u + S + 1 < 8 ? 1 : inc);
+            if constexpr (u == 7 - S) issue_sb(nsb, sb_inc);
+            if constexpr ((u & 1) == 1) offsets(X, co);
+            group_sb((u + 1) & 7);
+            form(0, r0, a0, b0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+        step(std::integral_constant<int, 7>{});
+    }
+    wait_vmcnt<0>();                                     // no DMA outstanding past the loop
+    mfma_result_pad();
+#pragma unroll
+    for (int i = 0; i < RI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) fold(i, j);
+
+    // Teams: team i takes over row tile i of every wave, adding the teams'
+    // sums in team order; they travel through LDS (the rings, free now).
+    auto mine = [&](int i) { return KW == 1 || i == team; };
+    if constexpr (KW > 1) {
+        static_assert(KW >= RI, "a team per row tile");
+        constexpr int CAP = KW == RI ? RI - 1 : RI;      // row tiles a team hands over, at most
+        f32x4_t* ex = reinterpret_cast<f32x4_t*>(&rings[0]);
+        static_assert((size_t)KW * Sh::NW * CAP * NJ * 4 * 64 * 16 <= sizeof(rings), "exchange area");
+        auto slot = [&](int k, int i) {
+            return (((k * Sh::NW + wave) * CAP + (KW == RI && i > k ? i - 1 : i)) * NJ) * 4 * 64 + lane;
+        };
+        lds_barrier();                                   // every wave is done with its ring
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            if (mine(i)) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    ex[slot(team, i) + (j * 4 + q) * 64] = (f32x4_t){acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                                    acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < RI; ++i) {
+            if (!mine(i)) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int k = 0; k < KW; ++k) {
+                        const f32x4_t own = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                             acc[i][j][4 * q + 3]};
+                        const f32x4_t v = k == i ? own : ex[slot(k, i) + (j * 4 + q) * 64];
+                        sum = k == 0 ? v : sum + v;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] = sum[r];
+                }
+        }
+    }
+
+    // ---- epilogue: lane l of a 32 x 32 tile holds rows (e/4)*8 + (l/32)*4 + e%4, column l%32 ----
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+        if (!mine(i)) continue;
+#pragma unroll
+        for (int j = 0; j < (NMAT == 2 ? 1 : NJ); ++j) {
+            const int cn = NMAT == 2 ? n0 + wn * 32 + col : n0 + wn * (32 * NJ) + j * 32 + col;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + (wm * RI + i) * 32 + (e >> 2) * 8 + h * 4 + (e & 3);
+                if (row >= M || cn >= N) continue;
+                const int64_t o = (int64_t)row * N + cn;
+                const float v = acc[i][j][e];
+                if (EPI == GEMM_STORE) {
+                    reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)f32_to_bf16(v);
+                } else if (EPI == GEMM_STORE_F32) {
+                    reinterpret_cast<float*>(p.y)[o] = v;
+                } else if (EPI == GEMM_RESIDUAL) {
+                    reinterpret_cast<uint16_t*>(p.y)[o] =
+                        (uint16_t)f32_to_bf16(bf16_to_f32(p.res[o]) + round_bf16(v));
+                } else {
+                    reinterpret_cast<uint16_t*>(p.y)[o] = (uint16_t)swiglu_bf16(v, acc[i][1][e]);
+                }
+            }
+        }
+    }
+}
+
+template <int EPI, int WR, int WC, int S, int KW>
+void launch_tile(const GemmArgs& a, unsigned blocks, hipStream_t st) {
+    hipLaunchKernelGGL((q4_gemm_ring_kernel<EPI, WR, WC, S, KW>), dim3(blocks), dim3(64 * WR * WC * KW), 0, st, a);
+}
+
+// Whether the ring kernel takes the product (whole eight-group blocks of K,
+// scale and bias rows 16-byte aligned, 32-bit byte offsets), and if so the
+// launch.  Few rows leave CUs idle and each block serial along K: the
+// smallest tile whose blocks stay within one per CU, on 4 (K % 2048 == 0) or
+// 2 (K % 1024 == 0) K teams, else 128 x 128 tiles, two blocks per CU.
+// Measured, us per call (M x N x K; 64 x 64 / 64 x 128 / 128 x 128, and the
+// kernel above, on 128 x 128 tiles throughout):
+//     77 x 4096 x 2048:  12.1 / 17.0 / 27.2,    33.0
+//    200 x 2048 x 6144:  26.7 / 39.2 / 71.0,    90.3
+//    300 x 4096 x 2048:  22.6 / 17.2 / 27.6,    33.3
+//   1024 x 2048 x 2048:  25.0 / 19.2 / 28.4,    34.2
+//    600 x 6144 x 2048:  44.1 / 34.7 / 29.1,    36.0
+//   1960 x 6144 x 2048: 131.7 / 101.8 / 80.0,   88.5
+//   2048 x 2048 x 6144: 110.8 / 87.1 / 78.9,    100.3
+// K = 512 has only one eight-group block for the ring's prologue to pay for
+// (77 x 4096 x 512: 11.8 against 11.1 us), so it stays on the kernel above.
+template <int EPI>
+bool launch_ring(const GemmArgs& a, hipStream_t st) {
+    auto a16 = [](const QMat& q) { return aligned(q.s, 16) && aligned(q.b, 16); };
+    const bool fits32 = (int64_t)a.M * a.K * 2 <= 0xFFFFFFFFLL && (int64_t)a.N * a.K / 2 <= 0xFFFFFFFFLL;
+    if (!fits32 || a.K % 512 != 0 || a.K < 1024 || !a16(a.A) || (EPI == GEMM_SWIGLU && !a16(a.B))) return false;
+    const int64_t cols = EPI == GEMM_SWIGLU ? 2 * (int64_t)a.N : a.N, cus = num_cus();
+    auto blocks = [&](int r, int c) { return (a.M + r - 1) / r * ((cols + c - 1) / c); };
+    const int teams = a.K % 2048 == 0 ? 4 : a.K % 1024 == 0 ? 2 : 1;
+    if constexpr (EPI != GEMM_SWIGLU) {                  // a wave pairs gate and up columns of one 128-column tile
+        const int64_t n = blocks(64, 64);
+        if (teams > 1 && n <= cus) {
+            if (teams == 4) launch_tile<EPI, 1, 1, 2, 4>(a, (unsigned)n, st);
+            else launch_tile<EPI, 1, 1, 4, 2>(a, (unsigned)n, st);
+            return true;
+        }
+    }
+    const int64_t n = blocks(64, 128);
+    if (teams > 1 && n <= cus) {
+        if (teams == 4) launch_tile<EPI, 1, 2, 2, 4>(a, (unsigned)n, st);
+        else launch_tile<EPI, 1, 2, 4, 2>(a, (unsigned)n, st);
+        return true;
+    }
+    launch_tile<EPI, 2, 2, 2, 1>(a, (unsigned)blocks(128, 128), st);
+    return true;
+}
+
+}  // namespace ring
+
 template <int EPI, bool NORM>
 int launch(const GemmArgs& a, hipStream_t st) {
     constexpr int BN = EPI == GEMM_SWIGLU ? 64 : 128;
@@ -702,6 +1147,9 @@ int launch(const GemmArgs& a, hipStream_t st) {
         if (NORM || !dma_ok) return -1;
         dma::launch_dma_auto<EPI>(a, st);
         return 0;
+    }
+    if constexpr (!NORM) {
+        if (ring::launch_ring<EPI>(a, st)) return 0;
     }
     if (NORM || !dma_ok)
         hipLaunchKernelGGL((q4_gemm_kernel<EPI, NORM>), dim3(blocks), dim3(kThreads), 0, st, a);

@@ -462,3 +462,38 @@ def test_mlp_residual_tile_edges(mq4, O, dev, M, K, N):
     rel = float(d.norm() / m.norm())
     print(f"identical {same:.5f}, rms(diff)/rms(mlp) {rel:.2e}")
     assert same >= 0.95 and rel <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 512, 1024), (64, 64, 2048), (65, 1000, 2048), (128, 4096, 2048),
+                                   (129, 8200, 2048), (192, 4104, 1024), (300, 4096, 1024), (257, 6144, 1536),
+                                   (520, 4100, 2048), (1100, 2052, 1024), (40, 33, 6144), (77, 4096, 512)])
+def test_gemm_ring_tiles(mq4, O, dev, M, N, K):
+    """The exact-operand GEMM at the edges of its tiles (64 x 64 and 64 x 128
+    with 4 or 2 K teams, 128 x 128; ragged rows and columns; K of 8, 16, 24,
+    32 and 96 groups), every epilogue: the fp32 result within GEMM_TOL_F32 of
+    the fp64 product, the bf16 store and the residual add exactly its
+    rounding, and the SwiGLU of the two products within one bf16 unit of the
+    sums' error (>= 98% of the bits: a pre-activation on a rounding boundary
+    moves with the order of its sums)."""
+    import torch
+    print(f"gemm ring tiles M={M} N={N} K={K}", flush=True)
+    (qa, _), (qb, _) = make(mq4, O, N, K, 1800, dev), make(mq4, O, N, K, 1801, dev)
+    x = mq4.fill_normal_bf16((M, K), mq4.STREAM_PREFILL + 8, 0.0, 1.0, device=dev)
+    res = mq4.fill_normal_bf16((M, N), mq4.STREAM_PREFILL + 9, 0.0, 1.0, device=dev)
+    ref = x.double() @ mq4.dequantize(*qa, dtype=torch.float32).double().t().contiguous()
+    y32 = mq4.quantized_matmul_f32(x, *qa)
+    err = float((y32.double() - ref).abs().max() / ref.square().mean().sqrt())
+    print(f"max |err| / rms {err:.2e}")
+    assert err <= GEMM_TOL_F32
+    guard = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=dev)
+    A, B = mq4.QuantizedTensor(*qa), mq4.QuantizedTensor(*qb)
+    y = mq4.qmatmul_residual(x, A, res, out=guard[:M])
+    assert torch.equal(mq4.qmatmul(x, A), y32.bfloat16())
+    assert torch.equal(y, (res.float() + y32.bfloat16().float()).bfloat16())
+    assert bool((guard[M] == 7.0).all()), "a row past M was written"
+    h = mq4.mlp_gate_up_silu(x, A, B)
+    hs = mq4.swiglu(mq4.qmatmul(x, A), mq4.qmatmul(x, B))
+    same = float((h.view(torch.int16) == hs.view(torch.int16)).float().mean())
+    print(f"swiglu identical {same:.5f}")
+    assert same >= 0.98
