@@ -92,6 +92,12 @@ __device__ __forceinline__ uint64_t fixed_mass(float s, float smax) {
     return (uint64_t)((double)expf(s - smax) * kFix + 0.5);
 }
 
+// Whether the masses are defined: with an infinite largest scaled value
+// (an infinite logit, or one over a tiny temperature) softmax is NaN
+// throughout, no element has a mass to compare with top_p, and the mask
+// leaves everything in.
+__device__ __forceinline__ bool mass_defined(float smax) { return fabsf(smax) <= 3.4028234663852886e38f; }
+
 // The Gumbel-perturbed value of kept element i (scaled value s) and its
 // 64-bit draw key: the float's order key in the high word, ~i in the low word
 // (the lowest index wins equal values).
@@ -304,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __rest
     // ---- top-p: keys above kstar masked, the first tie_keep ties at kstar kept ----
     uint32_t kstar = 0xffffu;
     int64_t tie_keep = -1;                             // -1: every element equal to kstar is kept
-    if (top_p > 0.0f && top_p < 1.0f) {
+    if (top_p > 0.0f && top_p < 1.0f && mass_defined(smax)) {
         for (int i = tid; i < 256; i += kThreads) mass[i] = 0;
         for (int i = tid; i < kWaves * 256; i += kThreads) (&wcnt[0][0])[i] = 0;
         __syncthreads();
@@ -718,7 +724,7 @@ __global__ __launch_bounds__(kCT) void chunk_draw_kernel(ChunkArgs a) {
     uint32_t kstar = 0xffffu;
     int64_t tie_keep = -1;
     uint32_t run = 0;                                  // ties at kstar before the current step
-    if (a.use_p) {
+    if (a.use_p && mass_defined(scaled_of(bf16_of_key(kmax), T))) {
         const uint64_t limit = a.sel[m].limit, before_hb = a.sel[m].before_hb;
         const uint32_t hbp = a.sel[m].hbp;
         reduce_bins(a.mass_lo + (size_t)m * a.P * 256, a.P, mass);

@@ -201,3 +201,21 @@ def test_chunked_and_single_workgroup_paths_agree(mq4, dev, M):
             want = S.keep_mask(bits, t, k, p, dtype=np.float64)
             if S.topp_margin(bits, t, k, p) > 1e-6:
                 assert np.array_equal(a_keep.astype(bool), want)
+
+
+@pytest.mark.parametrize("chunked", [True, False])
+def test_infinite_largest_value(mq4, dev, chunked):
+    """An infinite largest scaled value (an infinite logit, a row of -inf, a
+    tiny temperature) leaves softmax undefined, so top-p masks nothing (its
+    search found no element with a mass, and the chunked path read its tie
+    counts at that missing element); +inf is drawn, the lowest index first."""
+    rng = np.random.default_rng(7)
+    V = 16384
+    bits = gen_logits(rng, 4, V, "normal")
+    bits[1, [900, 9000]] = 0x7f80
+    bits[2] = 0xff80
+    print(f"sample infinite rows chunked={chunked}", flush=True)
+    idx, keep = c_sample(mq4, to_dev(bits, dev), 0.9, 0, 0.5, 3, chunked)
+    assert idx[1] == 900 and keep[1].all() and keep[2].all()
+    idx, keep = c_sample(mq4, to_dev(bits[:1], dev), 1e-38, 0, 0.5, 3, chunked)
+    assert keep.all() and np.isinf(S.scaled_logits(bits[:1], 1e-38, np.float32)[0, idx[0]])
