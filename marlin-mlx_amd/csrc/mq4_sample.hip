@@ -228,12 +228,12 @@ __device__ __forceinline__ void for_each_step(const uint16_t* __restrict__ row, 
     }
 }
 
+// Row m of `logits` by the whole workgroup of kThreads threads.
 template <int VEC>
-__global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __restrict__ logits, int64_t N, int64_t S,
-                                                          float temperature, int top_k, float top_p, uint64_t seed,
-                                                          uint32_t* __restrict__ idx, uint8_t* __restrict__ keep_out) {
+__device__ void sample_row(int64_t m, const uint16_t* __restrict__ logits, int64_t N, int64_t S, float temperature,
+                           int top_k, float top_p, uint64_t seed, uint32_t* __restrict__ idx,
+                           uint8_t* __restrict__ keep_out) {
 #pragma clang fp contract(off)
-    const int64_t m = blockIdx.x;
     const uint16_t* row = logits + m * N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ uint32_t hist[256];
@@ -426,6 +426,13 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __rest
     if (tid == 0) idx[m] = best ? argmax_key_index(best) : 0u;
 }
 
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __restrict__ logits, int64_t N, int64_t S,
+                                                          float temperature, int top_k, float top_p, uint64_t seed,
+                                                          uint32_t* __restrict__ idx, uint8_t* __restrict__ keep_out) {
+    sample_row<VEC>(blockIdx.x, logits, N, S, temperature, top_k, top_p, seed, idx, keep_out);
+}
+
 // ---------------------------------------------------------------------------
 // Chunked path for a few long rows (decode batches): row m is cut into P
 // chunks of C logits (C a multiple of kStep), one 256-thread workgroup each,
@@ -437,7 +444,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __rest
 //   chunk_mass_lo  the top-p high byte; mass and counts per low byte inside it
 //   chunk_draw     k*, the ties kept, this chunk's earlier ties; Gumbel-max
 //   chunk_final    the row's token from the chunks' best keys
-// Only the stages the parameters need are launched.  The integer sums,
+// Only the stages the parameters need are launched (top-k without a keep
+// mask takes the candidate lists below instead).  The integer sums,
 // thresholds and per-element draws are sample_kernel's, so the two paths give
 // identical tokens and keep masks.
 constexpr int kCT = 256;                    // threads per chunk workgroup
@@ -829,6 +837,293 @@ inline bool chunk_eligible(int64_t M, int64_t N) {
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// ---------------------------------------------------------------------------
+// Top-k on candidate lists, for the chunked rows when no keep mask is asked
+// for: two launches instead of the chain's six, whose stages each wait for
+// the previous one's partial histograms.  Latency bounds both forms: 248,320
+// logits, top-k 50 and top-p 0.9 take 27.6 us per sample_token call (8.6 us
+// and 19.4 us of kernels), 40.5 us on the chain (six stages of 3 to 13 us).
+//   topk_list   each chunk selects its own top_k largest keys (the ties of
+//               the last one included) in LDS, and writes them with their
+//               indices in index order.  The row's k-th largest key is at
+//               least every chunk's, so the row's kept elements are all on
+//               the lists.
+//   list_draw   one workgroup per row reads the lists (about top_k per
+//               chunk), selects the k-th largest key, keeps the elements from
+//               there on (in index order: chunk by chunk), and applies top-p
+//               and the draw to those few.
+// Keys, masses, thresholds, tie ranks and draws are sample_kernel's, so the
+// token is the same.  More candidates than a list or the LDS holds (ties)
+// take sample_row's passes over the row.
+constexpr int kListCap = 16384;             // candidates of a row in LDS (128 KB)
+constexpr int kListSteps = 4;               // steps of a chunk held in registers: C <= 4 kStep
+
+struct ListArgs {
+    const uint16_t* logits;
+    int64_t N, C;
+    int P;
+    float temperature;
+    int top_k;
+    float top_p;
+    uint64_t seed;
+    int use_p;
+    uint32_t* count;                        // [M][P]
+    int cap;                                // list entries per chunk
+    uint64_t* list;                         // [M][P][cap]: index << 16 | key
+    uint32_t* idx;
+};
+
+__global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
+    const int p = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t m = blockIdx.y;
+    const uint16_t* row = a.logits + m * a.N;
+    __shared__ uint32_t hist[256];
+    __shared__ uint32_t selk[2];
+    __shared__ uint32_t wsum[kListSteps][kCW];
+    const int64_t beg = (int64_t)p * a.C, end = beg + a.C < a.N ? beg + a.C : a.N;
+    const uint32_t need = end - beg < a.top_k ? (uint32_t)(end - beg) : (uint32_t)a.top_k;
+    uint4 q[kListSteps];
+#pragma unroll
+    for (int t = 0; t < kListSteps; ++t) {
+        const int64_t i0 = beg + (int64_t)t * kStep + tid * 8;
+        q[t] = i0 < end ? *reinterpret_cast<const uint4*>(row + i0) : make_uint4(0, 0, 0, 0);
+    }
+    // f(key, element) over this thread's logits of step t
+    auto each = [&](int t, auto&& f) {
+        if (beg + (int64_t)t * kStep + tid * 8 >= end) return;
+        const uint32_t w[4] = {q[t].x, q[t].y, q[t].z, q[t].w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f(bf16_order_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu), e);
+    };
+    hist[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> 8], 1u); });
+    __syncthreads();
+    if (tid < 64) select_top_bin(hist, need, selk);
+    __syncthreads();
+    const uint32_t hb = selk[0], above = selk[1];
+    hist[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kListSteps; ++t)
+        each(t, [&](uint32_t k, int) { if ((k >> 8) == hb) atomicAdd(&hist[k & 0xffu], 1u); });
+    __syncthreads();
+    if (tid < 64) select_top_bin(hist, need - above, selk);
+    __syncthreads();
+    const uint32_t kloc = (hb << 8) | selk[0];
+    // positions in index order: step, thread, element
+    uint32_t cnt[kListSteps], inc[kListSteps];
+#pragma unroll
+    for (int t = 0; t < kListSteps; ++t) {
+        uint32_t c = 0;
+        each(t, [&](uint32_t k, int) { c += k >= kloc ? 1u : 0u; });
+        cnt[t] = inc[t] = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(inc[t], d);
+            if (lane >= d) inc[t] += o;
+        }
+        if (lane == 63) wsum[t][wave] = inc[t];
+    }
+    __syncthreads();
+    uint64_t* list = a.list + (m * a.P + p) * a.cap;
+    uint32_t base = 0;
+#pragma unroll
+    for (int t = 0; t < kListSteps; ++t) {
+        uint32_t pre = 0, tot = 0;
+#pragma unroll
+        for (int w = 0; w < kCW; ++w) {
+            const uint32_t x = wsum[t][w];
+            pre += w < wave ? x : 0u;
+            tot += x;
+        }
+        uint32_t at = base + pre + inc[t] - cnt[t];
+        each(t, [&](uint32_t k, int e) {
+            if (k < kloc) return;
+            if (at < (uint32_t)a.cap) list[at] = ((uint64_t)(beg + (int64_t)t * kStep + tid * 8 + e) << 16) | k;
+            ++at;
+        });
+        base += tot;
+    }
+    // more ties than the list holds: the row takes the general path
+    if (tid == 0) a.count[m * a.P + p] = base <= (uint32_t)a.cap ? base : (uint32_t)kListCap + 1u;
+}
+
+// Exclusive prefix over the block of one count per thread; *total the sum.
+// tmp holds kWaves words; contains barriers.
+__device__ __forceinline__ uint32_t block_prefix(uint32_t c, uint32_t* tmp, uint32_t* total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t inc = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(inc, d);
+        if (lane >= d) inc += o;
+    }
+    __syncthreads();
+    if (lane == 63) tmp[wave] = inc;
+    __syncthreads();
+    uint32_t pre = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t x = tmp[w];
+        pre += w < wave ? x : 0u;
+        tot += x;
+    }
+    *total = tot;
+    return pre + inc - c;
+}
+
+__global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
+#pragma clang fp contract(off)
+    const int64_t m = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ uint64_t cand[kListCap];
+    __shared__ uint32_t hist[256];
+    __shared__ unsigned long long mass[256];
+    __shared__ uint64_t tmp[kWaves];
+    __shared__ uint32_t tmp32[kWaves];
+    __shared__ uint64_t sel[2];
+    __shared__ uint32_t selk[2];
+    __shared__ uint32_t off[kThreads + 1];
+    // ---- the chunks' lists, one after the other (P <= kThreads) ----
+    uint32_t L;
+    const uint32_t nc = tid < a.P ? a.count[m * a.P + tid] : 0u;
+    off[tid] = block_prefix(nc, tmp32, &L);
+    if (tid < 256) hist[tid] = 0;
+    __syncthreads();
+    if (L > (uint32_t)kListCap) {                      // block-uniform
+        const int64_t S = ((a.N + kWaves * 512 - 1) / (kWaves * 512)) * 512;
+        sample_row<8>(m, a.logits, a.N, S, a.temperature, a.top_k, a.top_p, a.seed, a.idx, nullptr);
+        return;
+    }
+    uint64_t mk = 0;
+    for (int p = wave; p < a.P; p += kWaves) {
+        const uint64_t* src = a.list + (m * a.P + p) * a.cap;
+        const uint32_t o = off[p], n = (p + 1 < a.P ? off[p + 1] : L) - o;
+        for (uint32_t i = lane; i < n; i += 64) {
+            const uint64_t v = src[i];
+            cand[o + i] = v;
+            const uint32_t k = (uint32_t)v & 0xffffu;
+            mk = k > mk ? k : mk;
+            atomicAdd(&hist[k >> 8], 1u);
+        }
+    }
+    const uint32_t kmax = (uint32_t)block_max_u64<kWaves>(mk, tmp);   // its barriers also complete hist and cand
+    // ---- the k-th largest key (the lists hold at least top_k elements) ----
+    if (wave == 0) select_top_bin(hist, (uint32_t)a.top_k, selk);
+    __syncthreads();
+    const uint32_t hb = selk[0], above = selk[1];
+    if (tid < 256) hist[tid] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < L; i += kThreads) {
+        const uint32_t k = (uint32_t)cand[i] & 0xffffu;
+        if ((k >> 8) == hb) atomicAdd(&hist[k & 0xffu], 1u);
+    }
+    __syncthreads();
+    if (wave == 0) select_top_bin(hist, (uint32_t)a.top_k - above, selk);
+    __syncthreads();
+    uint32_t kmin = (hb << 8) | selk[0];
+    if (kmin == 0) kmin = 1;
+    if (kmax < kmin) {                                 // nothing but NaN
+        if (tid == 0) a.idx[m] = 0u;
+        return;
+    }
+    // ---- the elements from there on, in index order, to the front of cand ----
+    constexpr int kPer = kListCap / kThreads;
+    uint32_t F;
+    {
+        const uint32_t per = (L + kThreads - 1) / kThreads, b = tid * per;
+        uint64_t v[kPer];
+        uint32_t c = 0;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            v[e] = (uint32_t)e < per && b + e < L ? cand[b + e] : 0ull;
+            c += ((uint32_t)v[e] & 0xffffu) >= kmin ? 1u : 0u;
+        }
+        uint32_t at = block_prefix(c, tmp32, &F);      // its barriers: every read is done
+#pragma unroll
+        for (int e = 0; e < kPer; ++e)
+            if (((uint32_t)v[e] & 0xffffu) >= kmin) cand[at++] = v[e];
+    }
+    __syncthreads();
+    const float T = a.temperature;
+    uint32_t kstar = 0xffffu;
+    int64_t tie_keep = -1;                             // -1: every element equal to kstar is kept
+    const float smax = scaled_of(bf16_of_key(kmax), T);
+    if (a.use_p && mass_defined(smax)) {
+        if (tid < 256) mass[tid] = 0;
+        __syncthreads();
+        uint64_t z = 0;
+        for (uint32_t i = tid; i < F; i += kThreads) {
+            const uint32_t k = (uint32_t)cand[i] & 0xffffu;
+            const uint64_t f = fixed_mass(scaled_of(bf16_of_key(k), T), smax);
+            z += f;
+            if (f) atomicAdd(&mass[k >> 8], (unsigned long long)f);
+        }
+        const uint64_t Z = block_sum_u64<kWaves>(z, tmp);      // its barriers also complete mass
+        const uint64_t limit = (uint64_t)((double)a.top_p * (double)Z);
+        if (wave == 0) select_mass_bin(mass, 0, limit, sel);
+        __syncthreads();
+        const uint32_t hbp = (uint32_t)sel[0];
+        const uint64_t before_hb = sel[1];
+        __syncthreads();
+        if (tid < 256) mass[tid] = 0;
+        __syncthreads();
+        for (uint32_t i = tid; i < F; i += kThreads) {
+            const uint32_t k = (uint32_t)cand[i] & 0xffffu;
+            if ((k >> 8) != hbp) continue;
+            const uint64_t f = fixed_mass(scaled_of(bf16_of_key(k), T), smax);
+            if (f) atomicAdd(&mass[k & 0xffu], (unsigned long long)f);
+        }
+        __syncthreads();
+        if (wave == 0) select_mass_bin(mass, before_hb, limit, sel);
+        __syncthreads();
+        const uint64_t before_k = sel[1];
+        kstar = (hbp << 8) | (uint32_t)sel[0];
+        const uint64_t fe = fixed_mass(scaled_of(bf16_of_key(kstar), T), smax);
+        tie_keep = (int64_t)((limit - before_k) / fe) + 1;
+    }
+    // ---- Gumbel-max over the kept elements, each thread a run of them ----
+    const uint32_t per = (F + kThreads - 1) / kThreads, b = tid * per, e1 = b + per < F ? b + per : F;
+    uint32_t ties = 0, all;
+    for (uint32_t i = b; i < e1; ++i) ties += ((uint32_t)cand[i] & 0xffffu) == kstar ? 1u : 0u;
+    int64_t below = (int64_t)block_prefix(ties, tmp32, &all);  // ties at kstar before this run
+    uint64_t best = 0;
+    for (uint32_t i = b; i < e1; ++i) {
+        const uint64_t v = cand[i];
+        const uint32_t k = (uint32_t)v & 0xffffu;
+        bool keep = k <= kstar;
+        if (tie_keep >= 0 && k == kstar) {
+            keep = keep && below < tie_keep;
+            ++below;
+        }
+        if (!keep) continue;
+        float val;
+        const uint64_t key = draw_key(scaled_of(bf16_of_key(k), T), a.seed, m, (int64_t)(v >> 16), &val);
+        best = key > best ? key : best;
+    }
+    best = block_max_u64<kWaves>(best, tmp);
+    if (tid == 0) a.idx[m] = best ? argmax_key_index(best) : 0u;
+}
+
+// Chunks of the list path: the chain's, made larger until top_k (and some
+// ties) of every chunk fit the LDS list; false if they do not.
+inline bool list_shape(int64_t M, int64_t N, int top_k, int* P, int64_t* C) {
+    chunk_shape(M, N, P, C);
+    while (*C <= kListSteps * kStep) {
+        *P = (int)((N + *C - 1) / *C);
+        if (*P <= kThreads && (int64_t)*P * (top_k + 16) <= kListCap) return true;
+        *C *= 2;
+    }
+    return false;
+}
+// Workspace: a count per chunk (at most kThreads), and 2 kListCap entries per
+// row, shared evenly by its chunks (at least twice top_k + 16 each).
+inline size_t list_bytes(int64_t M) {
+    return align256((size_t)M * kThreads * 4) + (size_t)M * 2 * kListCap * 8;
+}
+
 // Workspace carve-up of the chunked path; returns the bytes needed.
 inline size_t chunk_layout(int64_t M, int P, char* base, ChunkArgs* a) {
     const size_t mp = (size_t)M * P, bins = mp * 256;
@@ -870,7 +1165,8 @@ extern "C" size_t mq4_sample_workspace_size(int64_t M, int64_t N) {
     int P;
     int64_t C;
     smp::chunk_shape(M, N, &P, &C);
-    return smp::chunk_layout(M, P, nullptr, nullptr);
+    const size_t chain = smp::chunk_layout(M, P, nullptr, nullptr), lists = smp::list_bytes(M);
+    return chain > lists ? chain : lists;
 }
 
 extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, float temperature, int top_k,
@@ -906,6 +1202,24 @@ extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, flo
         a.use_p = temperature > 0.0f && top_p > 0.0f && top_p < 1.0f;
         a.idx = idx;
         a.keep = keep;
+        smp::ListArgs l{};
+        if (a.use_k && !keep && smp::list_shape(M, N, top_k, &l.P, &l.C)) {
+            l.logits = logits;
+            l.N = N;
+            l.temperature = temperature;
+            l.top_k = top_k;
+            l.top_p = top_p;
+            l.seed = seed;
+            l.use_p = a.use_p;
+            l.idx = idx;
+            l.count = static_cast<uint32_t*>(workspace);
+            l.list = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + smp::align256((size_t)M * smp::kThreads * 4));
+            const int64_t cap = 2 * smp::kListCap / l.P;
+            l.cap = (int)(cap < l.C ? cap : l.C);
+            hipLaunchKernelGGL(smp::topk_list_kernel, dim3((unsigned)l.P, (unsigned)M), dim3(smp::kCT), 0, st, l);
+            hipLaunchKernelGGL(smp::list_draw_kernel, dim3((unsigned)M), dim3(smp::kThreads), 0, st, l);
+            return launch_status(what);
+        }
         const dim3 grid((unsigned)a.P, (unsigned)M);
         if (a.use_k || a.use_p) hipLaunchKernelGGL(smp::chunk_stats_kernel, grid, dim3(smp::kCT), 0, st, a);
         if (a.use_k) hipLaunchKernelGGL(smp::chunk_topk_kernel, grid, dim3(smp::kCT), 0, st, a);

@@ -219,3 +219,36 @@ def test_infinite_largest_value(mq4, dev, chunked):
     assert idx[1] == 900 and keep[1].all() and keep[2].all()
     idx, keep = c_sample(mq4, to_dev(bits[:1], dev), 1e-38, 0, 0.5, 3, chunked)
     assert keep.all() and np.isinf(S.scaled_logits(bits[:1], 1e-38, np.float32)[0, idx[0]])
+
+
+@pytest.mark.parametrize("M,V", [(1, 8192), (1, 8200), (3, 10248), (1, 151936), (4, 248320), (32, 65536), (128, 8192)])
+def test_candidate_lists_agree_with_single_workgroup(mq4, dev, M, V):
+    """Top-k without a keep mask on candidate lists against the one-workgroup
+    path, token for token: odd last chunks, ties (lists that overflow, rows of
+    one value), infinities, NaN, a row of NaN, the lowest finite value, top_k
+    from 1 past a chunk's size (the chain), with and without top-p."""
+    rng = np.random.default_rng(300 + M + V)
+    bits = gen_logits(rng, M, V, "normal")
+    bits[-1, : V // 2] = gen_logits(rng, 1, V // 2, "ties")[0]
+    bits[0, rng.integers(0, V, 40)] = 0x7fc0                 # NaN
+    bits[0, rng.integers(0, V, 40)] = 0xff80                 # -inf
+    if M > 2:
+        bits[1] = 0x4000                                     # one value
+        bits[2] = 0x7fc0                                     # nothing but NaN
+    if M > 3:
+        bits[3] = 0xff7f                                     # the lowest finite value, and three others
+        bits[3, [5, 6000, V - 1]] = [0x4100, 0x4110, 0x7f80]
+    x = to_dev(bits, dev)
+    L = mq4.lib()
+    ws = torch.full((L.mq4_sample_workspace_size(M, V),), 0xAB, dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    for t, k, p in [(1.0, 1, 1.0), (0.7, 50, 0.9), (1.3, 7, 0.05), (0.5, 200, 1.0), (1.0, 200, 0.5), (0.8, 500, 0.95),
+                    (0.9, 3000, 0.9), (1.0, V - 1, 1.0)]:
+        print(f"lists M={M} V={V} t={t} k={k} p={p}", flush=True)
+        got = []
+        for w, n in ((ws.data_ptr(), ws.numel()), (0, 0)):
+            idx = torch.full((M,), -7, dtype=torch.int32, device=dev)
+            rc = L.mq4_sample_bf16(x.data_ptr(), M, V, t, k, p, 1234 + k, idx.data_ptr(), None, w or None, n, stream)
+            assert rc == 0, L.mq4_last_error()
+            got.append(idx.cpu().numpy())
+        assert np.array_equal(got[0], got[1]), (t, k, p, np.nonzero(got[0] != got[1])[0][:8])
