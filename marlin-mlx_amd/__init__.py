@@ -134,12 +134,18 @@ def _check(rc: int) -> None:
         raise MQ4Error(rc, lib().mq4_last_error().decode())
 
 
-def _stream(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# The wrappers run in front of kernels of a few microseconds, so what they
+# call per launch is kept short: a one-token 512 x 2048 qmatmul takes 7.7 us
+# of host time (10.2 with a Stream object and a c_void_p per argument).  The
+# foreign functions' argument types convert plain ints.
+
+def _stream(device):
+    """The raw handle of the current stream of a tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: torch.Tensor | None):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def _need(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
@@ -149,7 +155,7 @@ def _need(t: torch.Tensor, dtype, name: str) -> torch.Tensor:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
     if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def _check_weight(fn: str, wq: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, K: int,
@@ -158,9 +164,10 @@ def _check_weight(fn: str, wq: torch.Tensor, scales: torch.Tensor, biases: torch
     of K features (what mx::quantized_matmul validates): wq int32 [N, K*bits/32],
     scales and biases bf16 [N, K/group_size].  Returns N.  Checked before any
     pointer reaches the C ABI, which only sees raw addresses."""
-    for t, name in ((wq, "weight"), (scales, "scales"), (biases, "biases")):
-        if not isinstance(t, torch.Tensor):
-            raise TypeError(f"{fn}: {name} must be a torch.Tensor")
+    if not (isinstance(wq, torch.Tensor) and isinstance(scales, torch.Tensor) and isinstance(biases, torch.Tensor)):
+        for t, name in ((wq, "weight"), (scales, "scales"), (biases, "biases")):
+            if not isinstance(t, torch.Tensor):
+                raise TypeError(f"{fn}: {name} must be a torch.Tensor")
     if wq.dtype != torch.int32:
         raise TypeError(f"{fn}: packed weight must be int32 (uint32 words), got {wq.dtype}")
     if scales.dtype != torch.bfloat16 or biases.dtype != torch.bfloat16:
@@ -174,12 +181,12 @@ def _check_weight(fn: str, wq: torch.Tensor, scales: torch.Tensor, biases: torch
                                   f"(got group_size={group_size}, bits={bits})")
     if K % group_size != 0 or (K * bits) % 32 != 0:
         raise ValueError(f"{fn}: K={K} is not a multiple of group_size={group_size}")
-    N = wq.shape[0]
-    if wq.shape[1] != K * bits // 32:
+    N, words = wq.shape
+    if words != K * bits // 32:
         raise ValueError(f"{fn}: input has K={K} features but the weight holds "
-                         f"{wq.shape[1] * 32 // bits} (shape {tuple(wq.shape)})")
+                         f"{words * 32 // bits} (shape {tuple(wq.shape)})")
     want = (N, K // group_size)
-    if tuple(scales.shape) != want or tuple(biases.shape) != want:
+    if scales.shape != want or biases.shape != want:
         raise ValueError(f"{fn}: scales/biases must be {want}, got {tuple(scales.shape)} and "
                          f"{tuple(biases.shape)}")
     return N
@@ -277,8 +284,7 @@ def dequantize(wq: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
 def _mk(x: torch.Tensor, N: int):
     K = x.shape[-1]
     M = x.numel() // K
-    y = torch.empty((*x.shape[:-1], N), dtype=torch.bfloat16, device=x.device)
-    return M, K, y
+    return M, K, x.new_empty((*x.shape[:-1], N))
 
 
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
@@ -531,7 +537,7 @@ def lm_head_argmax(hidden: torch.Tensor, w: QuantizedTensor, return_logits: bool
         return (idx, logits) if return_logits else idx
     L = lib()
     ws_bytes = L.mq4_lm_head_argmax_workspace_size(M, N)
-    ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=hidden.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=hidden.device)     # partial keys, written before they are read
     wargs = (_ptr(w.weight), _ptr(w.scales), _ptr(w.biases), N, _ptr(idx), _ptr(logits), _ptr(ws), ws_bytes,
              _stream(hidden.device))
     if norm_weight is None:
