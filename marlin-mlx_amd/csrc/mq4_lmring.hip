@@ -252,6 +252,230 @@ __global__ __launch_bounds__(kThreads) void lm_ring_kernel(Params p) {
 
 }  // namespace lmr
 
+// ---- 9-16 rows: a wave per tile ----
+//
+// lm_ring_kernel splits every tile's K over the 8 waves, so each tile costs
+// each of them a barrier, a round of partials through LDS and a share of the
+// sum: 220 VALU per wave and tile, 108 of them unpacking and folding, and the
+// VALU bounds it (72 us at 16 rows, 248,320 x 2048).  With the normalized,
+// pair-ordered activations of all 16 rows in LDS (64 KB, read back 16 bytes
+// per lane and MFMA) a wave runs a whole tile alone: no barrier in the loop,
+// and the eight 4-group partials are added in registers, in the same order,
+// so the logits keep their bits.  Each wave streams its own tiles, one
+// 128-byte line of the 16 rows (4 groups) per ring stage, kR stages in flight
+// (73 KB per CU).  Kernel time at 16 rows with the weights partly in the
+// last-level cache 72.2 -> 55.7 us (1010 VALU per tile instead of 1760); a
+// call on weights read from memory 74.8 -> 70.2 us (100,003 columns 37.3 ->
+// 35.8), memory-bound now: waves starting on different lines, six stages or
+// 16 waves per CU measured no better.  Up to 8 rows, with half the logits to
+// write, lm_ring_kernel is as fast or faster (100,003 columns 33.5 against
+// 34.3 us at 8 rows), so it keeps those.
+namespace lmw {
+
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+constexpr int K = 2048, G = K / 64;    // 32 groups
+constexpr int kLines = K / 256;        // 128-byte lines per packed row (4 groups each)
+constexpr int kR = 4;                  // stages in flight per wave; divides kLines
+constexpr int kDmaPerStage = 3;        // two 1 KB line blocks, one scale/bias block
+constexpr int kMinM = 9, kMaxM = 16;
+
+struct alignas(16) Smem {
+    uint4 x[G][2][64];                 // activations, MFMA A operand: [group][half][lane] (64 KB)
+    mf::f32x4_t xs[G][4];              // group sums of rows 4 kq + i (2 KB)
+    uint4 w[kWaves][kR][2][64];        // each wave's line blocks, rows 0-7 and 8-15 (64 KB)
+    uint32_t sb[kWaves][kR][64];       // each wave's scales (dwords 0-31) and biases (32-63)
+    float ss[kWaves][kMaxM];
+    uint64_t best[kWaves][kMaxM];
+};
+
+template <bool NORM>
+__global__ __launch_bounds__(kThreads, 2) void lm_wave_kernel(lmr::Params p) {
+#pragma clang fp contract(off)
+    __shared__ Smem sm;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15, kq = lane >> 4;
+    const int M = p.M, N = p.N;
+    // Rows in R full rounds of 16-row tiles, and the remaining rem rows as
+    // one short tile of at most q = ceil(rem / W) rows per wave, taken first
+    // (as in lm_ring_kernel); its missing rows repeat its last row.
+    const int W = (int)gridDim.x * kWaves, gw = (int)blockIdx.x * kWaves + wave;
+    const int R = N / (16 * W), rem = N - R * 16 * W;
+    const int q = (rem + W - 1) / W;
+    const int rshort = R * 16 * W + gw * q;
+    const int nshort = rem == 0 ? 0 : (N - rshort < q ? (N - rshort > 0 ? N - rshort : 0) : q);
+    const int S = nshort > 0 ? 1 : 0;
+    const int T = R + S;
+    auto tile_n0 = [&](int j) { return j < S ? rshort : 16 * (gw + (j - S) * W); };
+    auto tile_rows = [&](int j) { return j < S ? nshort : 16; };
+
+    // ---- the ring: line l of tile j -> stage l % kR ----
+    const uint32_t w_lds = stage::lds_addr(&sm.w[wave][0][0][0]), sb_lds = stage::lds_addr(&sm.sb[wave][0][0]);
+    // byte offsets of this lane's chunks from the tile's first row (rows past
+    // the tile's last repeat it)
+    uint32_t woff[2], sboff;
+    auto tile_offsets = [&](int j) {
+        const int last = tile_rows(j) - 1;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int sl = 64 * b + lane, row = sl >> 3, u = stage::stage_chunk(sl, row);
+            woff[b] = (uint32_t)((row < last ? row : last) * (K / 2) + 16 * u);
+        }
+        const int r = (lane & 31) >> 1;
+        sboff = (uint32_t)((r < last ? r : last) * (G * 2) + 4 * (lane & 1));
+    };
+    auto issue = [&](int64_t n0, int l, int slot) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            stage::dma16_m0(reinterpret_cast<const char*>(p.A.wq) + n0 * (K / 2) + 128 * l, woff[b],
+                            w_lds + (uint32_t)(slot * 2048 + b * 1024));
+        const char* src = lane < 32 ? reinterpret_cast<const char*>(p.A.s) : reinterpret_cast<const char*>(p.A.b);
+        stage::dma4_m0(src + n0 * (G * 2) + 8 * l + sboff, sb_lds + (uint32_t)(slot * 256));
+    };
+
+    // ---- activations: this wave's 4 groups of the 16 rows, normalized, in
+    // pair order, with their group sums (the values lm_ring_kernel holds) ----
+    constexpr int GWA = G / kWaves;
+    const int g0 = wave * GWA;
+    uint4 xa[GWA][2], nwv[GWA][2];
+    {
+        const int mm = c16 < M ? c16 : M - 1;          // rows >= M repeat row M - 1, never read back
+#pragma unroll
+        for (int gi = 0; gi < GWA; ++gi) {
+            const uint4* src = reinterpret_cast<const uint4*>(p.x + (int64_t)mm * K + 64 * (g0 + gi) + 16 * kq);
+            xa[gi][0] = src[0];
+            xa[gi][1] = src[1];
+        }
+        if constexpr (NORM) {
+#pragma unroll
+            for (int gi = 0; gi < GWA; ++gi) {
+                const uint4* src = reinterpret_cast<const uint4*>(p.norm + 64 * (g0 + gi) + 16 * kq);
+                nwv[gi][0] = src[0];
+                nwv[gi][1] = src[1];
+            }
+            float s = 0.0f;
+#pragma unroll
+            for (int gi = 0; gi < GWA; ++gi) {
+                mf::sumsq4(s, xa[gi][0]);
+                mf::sumsq4(s, xa[gi][1]);
+            }
+            s += __shfl_xor(s, 16);
+            s += __shfl_xor(s, 32);
+            if (kq == 0) sm.ss[wave][c16] = s;
+        }
+    }
+    wait_vmcnt<0>();                                   // tracked loads are in before any DMA is issued
+    if (T > 0) {
+        tile_offsets(0);
+#pragma unroll
+        for (int l = 0; l < kR; ++l) issue(tile_n0(0), l, l);
+    }
+    lds_barrier();                                     // sums of squares
+    const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const mf::f32x4_t zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (NORM) {
+        float tot = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) tot += sm.ss[w][c16];
+        const float r = rms_inv(tot, K, p.eps);
+#pragma unroll
+        for (int gi = 0; gi < GWA; ++gi)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint4 v = xa[gi][h], w = nwv[gi][h];
+                xa[gi][h] = make_uint4(norm_word(v.x, w.x, r), norm_word(v.y, w.y, r), norm_word(v.z, w.z, r),
+                                       norm_word(v.w, w.w, r));
+            }
+    }
+#pragma unroll
+    for (int gi = 0; gi < GWA; ++gi) {
+        xa[gi][0] = mf::pair_order(xa[gi][0]);
+        xa[gi][1] = mf::pair_order(xa[gi][1]);
+        const mf::f32x4_t X = mf::mfma16(xa[gi][1], ones, mf::mfma16(xa[gi][0], ones, zero4));
+        sm.x[g0 + gi][0][lane] = xa[gi][0];
+        sm.x[g0 + gi][1][lane] = xa[gi][1];
+        if (c16 == 0) sm.xs[g0 + gi][kq] = X;          // every column holds the sums of rows 4 kq + i
+    }
+    lds_barrier();
+
+    uint64_t best[4] = {0, 0, 0, 0};                   // rows 4 kq + i, this lane's column
+    for (int j = 0; j < T; ++j) {
+        const int n0 = tile_n0(j);
+        const bool more = j + 1 < T;
+        const int64_t nn = more ? tile_n0(j + 1) : n0; // past the end: lines of this tile again, not used
+        float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int l = 0; l < kLines; ++l) {
+            const int slot = l % kR;
+            // lines l + 1 .. l + kR - 1 may stay in flight (logit stores in
+            // the queue only make the wait stricter)
+            wait_vmcnt<(kR - 1) * kDmaPerStage>();
+            const uint2* wl = reinterpret_cast<const uint2*>(&sm.w[wave][slot][0][0]);
+            const uint2 sw = *reinterpret_cast<const uint2*>(&sm.sb[wave][slot][2 * c16]);
+            const uint2 bw = *reinterpret_cast<const uint2*>(&sm.sb[wave][slot][32 + 2 * c16]);
+            mf::f32x4_t acc = zero4;
+#pragma unroll
+            for (int gi = 0; gi < 4; ++gi) {
+                const uint2 wv = wl[2 * stage::stage_slot(c16, c16, 2 * gi + (kq >> 1)) + (kq & 1)];
+                const uint4 a0 = sm.x[4 * l + gi][0][lane], a1 = sm.x[4 * l + gi][1][lane];
+                const mf::f32x4_t X = sm.xs[4 * l + gi][kq];
+                const uint4 b0 = mf::unpack_word(wv.x), b1 = mf::unpack_word(wv.y);
+                const uint32_t s2 = gi < 2 ? sw.x : sw.y, b2 = gi < 2 ? bw.x : bw.y;
+                const float s = bf16_to_f32((gi & 1) ? (s2 >> 16) : (s2 & 0xffffu));
+                const float c = affine_c(s, (gi & 1) ? (b2 >> 16) : (b2 & 0xffffu));
+                const mf::f32x4_t P = mf::mfma16(a1, b1, mf::mfma16(a0, b0, zero4));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(s, P[i], __builtin_fmaf(c, X[i], acc[i]));
+            }
+            // the 8 partials of 4 groups in order, as the 8 waves' are added there
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[i] = l == 0 ? acc[i] : total[i] + acc[i];
+            // every read of this stage is done before its refill is issued
+            // (the sums as operands: the compiler would otherwise move every
+            // line's folds to the end of the tile, holding all products)
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(total[0]), "+v"(total[1]), "+v"(total[2]), "+v"(total[3])::"memory");
+            if (l + kR == kLines) tile_offsets(more ? j + 1 : j);
+            if (l + kR < kLines) issue(n0, l + kR, slot);
+            else issue(nn, l + kR - kLines, slot);
+        }
+        if (c16 < tile_rows(j)) {
+            const int n = n0 + c16;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 4 * kq + i;
+                if (m >= M) continue;
+                const uint32_t lb = f32_to_bf16(total[i]);
+                if (p.y) p.y[(int64_t)m * N + n] = (uint16_t)lb;
+                const uint64_t key = argmax_key(lb, (uint32_t)n);
+                best[i] = key > best[i] ? key : best[i];
+            }
+        }
+    }
+    wait_vmcnt<0>();                                   // no DMA outstanding past the loop
+
+    // ---- per-workgroup best key of each row: 16 columns, then the waves ----
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint64_t b = best[i];
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            const uint64_t o = shfl_xor_u64(b, off);
+            b = o > b ? o : b;
+        }
+        if (c16 == 0) sm.best[wave][4 * kq + i] = b;
+    }
+    __syncthreads();
+    if (tid < M) {
+        uint64_t b = sm.best[0][tid];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) b = sm.best[w][tid] > b ? sm.best[w][tid] : b;
+        p.partial[(int64_t)tid * kPartialStride + blockIdx.x] = b;
+    }
+}
+
+}  // namespace lmw
+
 // ---- 1-2 rows: the dot2 GEMV's arithmetic through the same kind of ring ----
 //
 // The dot2 GEMV (mq4_gemv.hip, K = 2048: one 16-byte slice per lane, 4 rows
@@ -465,9 +689,12 @@ int launch_lm_ring(const GemvParams& a, bool norm, hipStream_t st) {
             if (norm) hipLaunchKernelGGL((lmd::lm_ring_dot2_kernel<2, true>), g, bd, 0, st, p);
             else hipLaunchKernelGGL((lmd::lm_ring_dot2_kernel<2, false>), g, bd, 0, st, p);
         }
-    } else if (a.m_valid <= 16) {
+    } else if (a.m_valid < lmw::kMinM) {
         if (norm) hipLaunchKernelGGL((lmr::lm_ring_kernel<1, true>), g, b, 0, st, p);
         else hipLaunchKernelGGL((lmr::lm_ring_kernel<1, false>), g, b, 0, st, p);
+    } else if (a.m_valid <= lmw::kMaxM) {
+        if (norm) hipLaunchKernelGGL(lmw::lm_wave_kernel<true>, g, b, 0, st, p);
+        else hipLaunchKernelGGL(lmw::lm_wave_kernel<false>, g, b, 0, st, p);
     } else {
         if (norm) hipLaunchKernelGGL((lmr::lm_ring_kernel<2, true>), g, b, 0, st, p);
         else hipLaunchKernelGGL((lmr::lm_ring_kernel<2, false>), g, b, 0, st, p);

@@ -50,9 +50,13 @@ __device__ __forceinline__ void dma4_s(const void* base, uint32_t voff, const vo
                  :: "v"(voff), "s"(base), "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr(lds_dst))) : "memory");
 }
 
-// dma16_s with the wave-uniform LDS byte address (lds_addr) kept by the caller.
+// dma16_s and dma4 with the wave-uniform LDS byte address (lds_addr) kept by
+// the caller.
 __device__ __forceinline__ void dma16_m0(const void* base, uint32_t voff, uint32_t lds_dst) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(base), "{m0}"(lds_dst) : "memory");
+}
+__device__ __forceinline__ void dma4_m0(const void* src, uint32_t lds_dst) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" :: "v"(src), "{m0}"(lds_dst) : "memory");
 }
 
 __device__ __forceinline__ int stage_slot(int G, int row, int u) { return 8 * G + ((u - (row >> 1)) & 7); }

@@ -236,3 +236,28 @@ def test_lm_head_ring_small_m_rows_independent(mq4, O, dev, lm, M):
     ref64, refb = O.qmm_f64(hn, *qh)
     ulp = O.bf16_ulp_diff(to_host_u16(lg), refb)
     assert np.mean(ulp == 0) >= 0.98
+
+
+@pytest.mark.parametrize("M,N", [(8, 33000), (9, 15), (9, 33000), (12, 32768), (16, 32767), (16, 32769), (13, 100003)])
+def test_lm_head_wave_tiles(mq4, dev, M, N):
+    """From 9 to 16 rows a wave runs whole 16-row tiles of the lm_head by
+    itself (mq4_lmring.hip, lm_wave_kernel), below the 8-wave split: without
+    the norm the logits equal the plain product's, bit for bit; with it (whose
+    sum of squares is the lm_head kernels' own) those of 8-row calls, whose
+    rows are independent; the tokens are the first argmax.  At exactly one
+    tile per wave (32768 rows on 256 CUs), one row short of and past it, and
+    at fewer tiles than waves."""
+    import torch
+    print(f"lm_head wave tiles M={M} N={N}", flush=True)
+    qt = mq4.quantize_weight(mq4.fill_normal_bf16((N, H), 7300 + N, 0.0, 0.02, device=dev))
+    x = mq4.fill_normal_bf16((M, H), 3500 + M, 0.0, 2.0, device=dev)
+    nw = mq4.fill_normal_bf16((H,), 3600, 0.1, 0.02, device=dev)
+    idx, logits = mq4.lm_head_argmax(x, qt, return_logits=True)
+    ref = mq4.qmatmul(x, qt)
+    assert torch.equal(logits.view(torch.int16), ref.view(torch.int16)), "plain"
+    assert torch.equal(idx, mq4.argmax(logits))
+    idx, logits = mq4.lm_head_argmax(x, qt, return_logits=True, norm_weight=nw)
+    for r0 in {0, M - 8}:
+        _, part = mq4.lm_head_argmax(x[r0:r0 + 8].contiguous(), qt, return_logits=True, norm_weight=nw)
+        assert torch.equal(logits[r0:r0 + 8].view(torch.int16), part.view(torch.int16)), "norm"
+    assert torch.equal(idx, mq4.argmax(logits))
