@@ -152,13 +152,14 @@ __device__ __forceinline__ uint64_t block_max_u64(uint64_t v, uint64_t* tmp) {
     return t;
 }
 
-// Wave 0: over 256 count bins, the largest b with count(bins >= b) >= need
+// Wave 0: over 64 PER count bins, the largest b with count(bins >= b) >= need
 // (need >= 1 and the total >= need); out[0] = b, out[1] = count(bins > b).
+template <int PER = 4>
 __device__ void select_top_bin(const uint32_t* hist, uint32_t need, uint32_t* out) {
     const int lane = threadIdx.x & 63;
-    uint32_t h[4], t = 0;
+    uint32_t h[PER], t = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { h[j] = hist[4 * lane + j]; t += h[j]; }
+    for (int j = 0; j < PER; ++j) { h[j] = hist[PER * lane + j]; t += h[j]; }
     // inclusive suffix sum over lanes (lane l: sum of lanes >= l)
     uint32_t suf = t;
 #pragma unroll
@@ -169,8 +170,8 @@ __device__ void select_top_bin(const uint32_t* hist, uint32_t need, uint32_t* ou
     uint32_t above = suf - t;                // bins of lanes > l
     uint32_t cand = 0, cabove = 0;           // 1 + the largest bin of this lane meeting need
 #pragma unroll
-    for (int j = 3; j >= 0; --j) {
-        if (!cand && above + h[j] >= need) { cand = 4 * lane + j + 1; cabove = above; }
+    for (int j = PER - 1; j >= 0; --j) {
+        if (!cand && above + h[j] >= need) { cand = PER * lane + j + 1; cabove = above; }
         above += h[j];
     }
     const uint64_t best = wave_max_u64(((uint64_t)cand << 32) | cabove);
@@ -841,8 +842,8 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Top-k on candidate lists, for the chunked rows when no keep mask is asked
 // for: two launches instead of the chain's six, whose stages each wait for
 // the previous one's partial histograms.  Latency bounds both forms: 248,320
-// logits, top-k 50 and top-p 0.9 take 27.6 us per sample_token call (8.6 us
-// and 19.4 us of kernels), 40.5 us on the chain (six stages of 3 to 13 us).
+// logits, top-k 50 and top-p 0.9 take 27.1 us per sample_token call (7.4 us
+// and 18.3 us of kernels), 40.5 us on the chain (six stages of 3 to 13 us).
 //   topk_list   each chunk selects its own top_k largest keys (the ties of
 //               the last one included) in LDS, and writes them with their
 //               indices in index order.  The row's k-th largest key is at
@@ -855,8 +856,13 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Keys, masses, thresholds, tie ranks and draws are sample_kernel's, so the
 // token is the same.  More candidates than a list or the LDS holds (ties)
 // take sample_row's passes over the row.
-constexpr int kListCap = 16384;             // candidates of a row in LDS (128 KB)
+constexpr int kListCap = 15360;             // candidates of a row in LDS (120 KB)
 constexpr int kListSteps = 4;               // steps of a chunk held in registers: C <= 4 kStep
+// Radix digits of the lists' selections: 11 bits, then 5.  Logits share few
+// sign and exponent bits, and LDS atomics of a wave to one bin go one by one:
+// with 8-bit digits the first histogram filled two or three bins (list_draw
+// 19.4 -> 18.3 us, topk_list 8.6 -> 7.4).
+constexpr int kDigitBins = 2048, kDigitShift = 5;
 
 struct ListArgs {
     const uint16_t* logits;
@@ -877,7 +883,7 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
     const int p = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t m = blockIdx.y;
     const uint16_t* row = a.logits + m * a.N;
-    __shared__ uint32_t hist[256];
+    __shared__ uint32_t hist[kDigitBins];
     __shared__ uint32_t selk[2];
     __shared__ uint32_t wsum[kListSteps][kCW];
     const int64_t beg = (int64_t)p * a.C, end = beg + a.C < a.N ? beg + a.C : a.N;
@@ -895,23 +901,24 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) f(bf16_order_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu), e);
     };
-    hist[tid] = 0;
+#pragma unroll
+    for (int i = 0; i < kDigitBins / kCT; ++i) hist[i * kCT + tid] = 0;
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> 8], 1u); });
+    for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> kDigitShift], 1u); });
     __syncthreads();
-    if (tid < 64) select_top_bin(hist, need, selk);
+    if (tid < 64) select_top_bin<kDigitBins / 64>(hist, need, selk);
     __syncthreads();
     const uint32_t hb = selk[0], above = selk[1];
     hist[tid] = 0;
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < kListSteps; ++t)
-        each(t, [&](uint32_t k, int) { if ((k >> 8) == hb) atomicAdd(&hist[k & 0xffu], 1u); });
+        each(t, [&](uint32_t k, int) { if ((k >> kDigitShift) == hb) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], 1u); });
     __syncthreads();
     if (tid < 64) select_top_bin(hist, need - above, selk);
     __syncthreads();
-    const uint32_t kloc = (hb << 8) | selk[0];
+    const uint32_t kloc = (hb << kDigitShift) | selk[0];
     // positions in index order: step, thread, element
     uint32_t cnt[kListSteps], inc[kListSteps];
 #pragma unroll
@@ -979,7 +986,7 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     const int64_t m = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ uint64_t cand[kListCap];
-    __shared__ uint32_t hist[256];
+    __shared__ uint32_t hist[kDigitBins];
     __shared__ unsigned long long mass[256];
     __shared__ uint64_t tmp[kWaves];
     __shared__ uint32_t tmp32[kWaves];
@@ -990,7 +997,8 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     uint32_t L;
     const uint32_t nc = tid < a.P ? a.count[m * a.P + tid] : 0u;
     off[tid] = block_prefix(nc, tmp32, &L);
-    if (tid < 256) hist[tid] = 0;
+#pragma unroll
+    for (int i = 0; i < kDigitBins / kThreads; ++i) hist[i * kThreads + tid] = 0;
     __syncthreads();
     if (L > (uint32_t)kListCap) {                      // block-uniform
         const int64_t S = ((a.N + kWaves * 512 - 1) / (kWaves * 512)) * 512;
@@ -1006,24 +1014,24 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
             cand[o + i] = v;
             const uint32_t k = (uint32_t)v & 0xffffu;
             mk = k > mk ? k : mk;
-            atomicAdd(&hist[k >> 8], 1u);
+            atomicAdd(&hist[k >> kDigitShift], 1u);
         }
     }
     const uint32_t kmax = (uint32_t)block_max_u64<kWaves>(mk, tmp);   // its barriers also complete hist and cand
     // ---- the k-th largest key (the lists hold at least top_k elements) ----
-    if (wave == 0) select_top_bin(hist, (uint32_t)a.top_k, selk);
+    if (wave == 0) select_top_bin<kDigitBins / 64>(hist, (uint32_t)a.top_k, selk);
     __syncthreads();
     const uint32_t hb = selk[0], above = selk[1];
     if (tid < 256) hist[tid] = 0;
     __syncthreads();
     for (uint32_t i = tid; i < L; i += kThreads) {
         const uint32_t k = (uint32_t)cand[i] & 0xffffu;
-        if ((k >> 8) == hb) atomicAdd(&hist[k & 0xffu], 1u);
+        if ((k >> kDigitShift) == hb) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], 1u);
     }
     __syncthreads();
     if (wave == 0) select_top_bin(hist, (uint32_t)a.top_k - above, selk);
     __syncthreads();
-    uint32_t kmin = (hb << 8) | selk[0];
+    uint32_t kmin = (hb << kDigitShift) | selk[0];
     if (kmin == 0) kmin = 1;
     if (kmax < kmin) {                                 // nothing but NaN
         if (tid == 0) a.idx[m] = 0u;
