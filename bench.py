@@ -822,7 +822,8 @@ def bench_sampling(E, lm, norm_w, x0):
     _SAMPLING_LOGITS[:] = [logits]
     return {"workload": "sample_token over 248320 bf16 logits, M=1", "logit_bytes": 2 * VOCAB, "cases": out,
             "note": "stream-ordered chain: chunk stats, top-k select, top-p mass passes, Gumbel-max "
-                    "draw, final reduce (only the stages a case needs); HIP events around 200 back-to-back calls"}
+                    "draw, final reduce (only the stages a case needs; top-k with top-p runs as candidate lists "
+                    "and one draw); HIP events around 200 back-to-back calls"}
 
 
 def bench_pack(E, layers, lm):

@@ -840,7 +840,7 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // ---------------------------------------------------------------------------
 // Top-k on candidate lists, for the chunked rows when no keep mask is asked
-// for: two launches instead of the chain's six, whose stages each wait for
+// for (with top-p, or many rows): two launches instead of the chain's six, whose stages each wait for
 // the previous one's partial histograms.  Latency bounds both forms: 248,320
 // logits, top-k 50 and top-p 0.9 take 27.1 us per sample_token call (7.4 us
 // and 18.3 us of kernels), 40.5 us on the chain (six stages of 3 to 13 us).
@@ -857,6 +857,7 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // token is the same.  More candidates than a list or the LDS holds (ties)
 // take sample_row's passes over the row.
 constexpr int kListCap = 15360;             // candidates of a row in LDS (120 KB)
+constexpr int64_t kListMinChunks = 512;     // without top-p: chunks of a call above which lists pay
 constexpr int kListSteps = 4;               // steps of a chunk held in registers: C <= 4 kStep
 // Radix digits of the lists' selections: 11 bits, then 5.  Logits share few
 // sign and exponent bits, and LDS atomics of a wave to one bin go one by one:
@@ -1211,7 +1212,14 @@ extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, flo
         a.idx = idx;
         a.keep = keep;
         smp::ListArgs l{};
-        if (a.use_k && !keep && smp::list_shape(M, N, top_k, &l.P, &l.C)) {
+        // Lists where they save most: top-p as well (one row, top-k 20 / 50 /
+        // 200: 24.5 / 25.7 / 30.8 us against the chain's 39), or more chunks
+        // than two workgroups per CU (6 rows of 122 chunks: 21.8 / 23.1 / 28.1
+        // against 29.5).  Below that the chain of top-k alone is four short
+        // stages and as fast or faster (one row 19.7 us at every top_k, lists
+        // 20.7 / 22.0 at 20 / 50; 4 rows 24.6, lists 21.1 to 27.3).
+        const bool lists = a.use_k && !keep && (a.use_p || M * a.P > smp::kListMinChunks);
+        if (lists && smp::list_shape(M, N, top_k, &l.P, &l.C)) {
             l.logits = logits;
             l.N = N;
             l.temperature = temperature;
