@@ -229,12 +229,12 @@ __device__ __forceinline__ void for_each_step(const uint16_t* __restrict__ row, 
     }
 }
 
-// Row m of `logits` by the whole workgroup of kThreads threads.
 template <int VEC>
-__device__ void sample_row(int64_t m, const uint16_t* __restrict__ logits, int64_t N, int64_t S, float temperature,
-                           int top_k, float top_p, uint64_t seed, uint32_t* __restrict__ idx,
-                           uint8_t* __restrict__ keep_out) {
+__global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __restrict__ logits, int64_t N, int64_t S,
+                                                          float temperature, int top_k, float top_p, uint64_t seed,
+                                                          uint32_t* __restrict__ idx, uint8_t* __restrict__ keep_out) {
 #pragma clang fp contract(off)
+    const int64_t m = blockIdx.x;
     const uint16_t* row = logits + m * N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ uint32_t hist[256];
@@ -425,13 +425,6 @@ __device__ void sample_row(int64_t m, const uint16_t* __restrict__ logits, int64
     });
     best = block_max_u64<kWaves>(best, tmp);
     if (tid == 0) idx[m] = best ? argmax_key_index(best) : 0u;
-}
-
-template <int VEC>
-__global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __restrict__ logits, int64_t N, int64_t S,
-                                                          float temperature, int top_k, float top_p, uint64_t seed,
-                                                          uint32_t* __restrict__ idx, uint8_t* __restrict__ keep_out) {
-    sample_row<VEC>(blockIdx.x, logits, N, S, temperature, top_k, top_p, seed, idx, keep_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -840,24 +833,37 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // ---------------------------------------------------------------------------
 // Top-k on candidate lists, for the chunked rows when no keep mask is asked
-// for (with top-p, or many rows): two launches instead of the chain's six, whose stages each wait for
-// the previous one's partial histograms.  Latency bounds both forms: 248,320
-// logits, top-k 50 and top-p 0.9 take 27.1 us per sample_token call (7.4 us
-// and 18.3 us of kernels), 40.5 us on the chain (six stages of 3 to 13 us).
-//   topk_list   each chunk selects its own top_k largest keys (the ties of
-//               the last one included) in LDS, and writes them with their
-//               indices in index order.  The row's k-th largest key is at
-//               least every chunk's, so the row's kept elements are all on
-//               the lists.
+// for (with top-p, or many rows): two launches instead of the chain's six,
+// whose stages each wait for the previous one's partial histograms.  Latency
+// bounds both forms: 248,320 logits, top-k 50 and top-p 0.9 take 27.1 us per
+// sample_token call (7.4 us and 18.0 us of kernels), 40.5 us on the chain (six
+// stages of 3 to 13 us).
+//   topk_list   each chunk selects its own top_k largest keys in LDS, and
+//               writes them with their indices in index order.  The ties of
+//               the last one are all listed if they fit into top_k +
+//               kListTies entries; else the first kListTies, and of the rest
+//               the chunk writes their number and their best draw.  The row's
+//               k-th largest key is at least every chunk's, so it follows
+//               from the lists and these numbers, and every kept element is
+//               on a list or is one of the counted ties.
 //   list_draw   one workgroup per row reads the lists (about top_k per
 //               chunk), selects the k-th largest key, keeps the elements from
 //               there on (in index order: chunk by chunk), and applies top-p
-//               and the draw to those few.
+//               and the draw to those few.  Unlisted ties matter only where
+//               the row's k-th key is theirs (usually it is not: they are a
+//               masked stretch of the vocabulary): then as their number times
+//               one mass, and as their chunk's best draw.  If the top-p mask
+//               keeps only the first ties at that key and ends inside a chunk,
+//               that chunk is read again.
 // Keys, masses, thresholds, tie ranks and draws are sample_kernel's, so the
-// token is the same.  More candidates than a list or the LDS holds (ties)
-// take sample_row's passes over the row.
+// token is the same.  Per call, back to back, one row of 248,320 logits, top-k
+// 50 and top-p 0.9: normal logits 25.2 us, half of them masked 26.5, all but
+// 20 masked 30.5 (-inf) or 33.5 (-1e4), one value throughout 41.5; when a
+// chunk with too many ties sent its row to one workgroup's passes 25.2, 310,
+// 676 and 1234, on the chain 39.0, 39.9, 43.2 and 46.9.
 constexpr int kListCap = 15360;             // candidates of a row in LDS (120 KB)
 constexpr int64_t kListMinChunks = 512;     // without top-p: chunks of a call above which lists pay
+constexpr int kListTies = 16;               // list entries of a chunk beyond top_k
 constexpr int kListSteps = 4;               // steps of a chunk held in registers: C <= 4 kStep
 // Radix digits of the lists' selections: 11 bits, then 5.  Logits share few
 // sign and exponent bits, and LDS atomics of a wave to one bin go one by one:
@@ -874,19 +880,22 @@ struct ListArgs {
     float top_p;
     uint64_t seed;
     int use_p;
-    uint32_t* count;                        // [M][P]
+    uint64_t* info;                         // [M][P]: listed | last key << 16 | its ties not listed << 32
+    uint64_t* tie;                          // [M][P]: the best draw key of the ties not listed, if any
     int cap;                                // list entries per chunk
     uint64_t* list;                         // [M][P][cap]: index << 16 | key
     uint32_t* idx;
 };
 
 __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
+#pragma clang fp contract(off)
     const int p = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t m = blockIdx.y;
     const uint16_t* row = a.logits + m * a.N;
     __shared__ uint32_t hist[kDigitBins];
     __shared__ uint32_t selk[2];
     __shared__ uint32_t wsum[kListSteps][kCW];
+    __shared__ uint64_t tmp[kCW];
     const int64_t beg = (int64_t)p * a.C, end = beg + a.C < a.N ? beg + a.C : a.N;
     const uint32_t need = end - beg < a.top_k ? (uint32_t)(end - beg) : (uint32_t)a.top_k;
     uint4 q[kListSteps];
@@ -902,11 +911,17 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) f(bf16_order_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu), e);
     };
+    auto flat = [&](int t) { return q[t].x == (q[t].x >> 16) * 0x10001u && q[t].y == q[t].x && q[t].z == q[t].x && q[t].w == q[t].x; };
 #pragma unroll
     for (int i = 0; i < kDigitBins / kCT; ++i) hist[i * kCT + tid] = 0;
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> kDigitShift], 1u); });
+    for (int t = 0; t < kListSteps; ++t) {
+        // eight equal logits (a masked stretch) in one addition: the additions
+        // to one address go one by one
+        if (flat(t)) each(t, [&](uint32_t k, int e) { if (e == 0) atomicAdd(&hist[k >> kDigitShift], 8u); });
+        else each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> kDigitShift], 1u); });
+    }
     __syncthreads();
     if (tid < 64) select_top_bin<kDigitBins / 64>(hist, need, selk);
     __syncthreads();
@@ -914,29 +929,36 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
     hist[tid] = 0;
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < kListSteps; ++t)
-        each(t, [&](uint32_t k, int) { if ((k >> kDigitShift) == hb) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], 1u); });
+    for (int t = 0; t < kListSteps; ++t) {
+        const uint32_t n = flat(t) ? 8u : 1u;
+        each(t, [&](uint32_t k, int e) {
+            if ((k >> kDigitShift) == hb && (e == 0 || n == 1u)) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], n);
+        });
+    }
     __syncthreads();
     if (tid < 64) select_top_bin(hist, need - above, selk);
     __syncthreads();
     const uint32_t kloc = (hb << kDigitShift) | selk[0];
-    // positions in index order: step, thread, element
+    const uint32_t over = above + selk[1];             // keys above kloc: fewer than need, so than cap
+    // positions in index order: step, thread, element.  Two counts of at most
+    // C = 8192 in a word: keys above kloc, and ties << 16.
     uint32_t cnt[kListSteps], inc[kListSteps];
 #pragma unroll
     for (int t = 0; t < kListSteps; ++t) {
         uint32_t c = 0;
-        each(t, [&](uint32_t k, int) { c += k >= kloc ? 1u : 0u; });
+        each(t, [&](uint32_t k, int) { c += k > kloc ? 1u : k == kloc ? 0x10000u : 0u; });
         cnt[t] = inc[t] = c;
+        if (beg + (int64_t)t * kStep < end) {          // block-uniform: not past the chunk
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t o = __shfl_up(inc[t], d);
-            if (lane >= d) inc[t] += o;
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t o = __shfl_up(inc[t], d);
+                if (lane >= d) inc[t] += o;
+            }
         }
         if (lane == 63) wsum[t][wave] = inc[t];
     }
     __syncthreads();
-    uint64_t* list = a.list + (m * a.P + p) * a.cap;
-    uint32_t base = 0;
+    uint32_t total = 0;                                // both counts of the steps before, then of the chunk
 #pragma unroll
     for (int t = 0; t < kListSteps; ++t) {
         uint32_t pre = 0, tot = 0;
@@ -946,16 +968,58 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
             pre += w < wave ? x : 0u;
             tot += x;
         }
-        uint32_t at = base + pre + inc[t] - cnt[t];
-        each(t, [&](uint32_t k, int e) {
-            if (k < kloc) return;
-            if (at < (uint32_t)a.cap) list[at] = ((uint64_t)(beg + (int64_t)t * kStep + tid * 8 + e) << 16) | k;
-            ++at;
-        });
-        base += tot;
+        cnt[t] = total + pre + inc[t] - cnt[t];        // both counts before this thread's logits of step t
+        total += tot;
     }
-    // more ties than the list holds: the row takes the general path
-    if (tid == 0) a.count[m * a.P + p] = base <= (uint32_t)a.cap ? base : (uint32_t)kListCap + 1u;
+    const uint32_t ties = total >> 16;
+    // All of the ties are listed if they fit, else the first few.
+    const uint32_t fit = (uint32_t)a.cap - over;
+    const uint32_t room = ties <= fit ? fit : (uint32_t)kListTies;   // then cap = top_k + kListTies
+    const uint32_t left = ties > room ? ties - room : 0u;       // block-uniform
+    uint64_t* list = a.list + (m * a.P + p) * a.cap;
+    // f(key, element, keys above kloc before it, ties before it) over the
+    // logits from kloc up, in this thread's order
+    auto each_top = [&](auto&& f) {
+#pragma unroll
+        for (int t = 0; t < kListSteps; ++t) {
+            uint32_t at = cnt[t];
+            each(t, [&](uint32_t k, int e) {
+                if (k < kloc) return;
+                f(k, beg + (int64_t)t * kStep + tid * 8 + e, at & 0xffffu, at >> 16);
+                at += k > kloc ? 1u : 0x10000u;
+            });
+        }
+    };
+    each_top([&](uint32_t k, int64_t i, uint32_t g, uint32_t r) {
+        if (k > kloc || r < room) list[g + (r < room ? r : room)] = ((uint64_t)i << 16) | k;
+    });
+    uint64_t best = 0;
+    if (left) {
+        // The best draw of the ties not listed.  Not needed for NaN (never
+        // kept); where the Gumbel noise (below 2^5) is lost in the value, as
+        // the listed ties come first then; nor for a value 50 below the
+        // chunk's largest, when it cannot win: the largest element that top-p
+        // keeps has a mass of at least 2^-41 of the largest one's, so its
+        // value is within 28.5 of that, and noise lies in (-3, kGumbelMax).
+        uint64_t mk = 0;
+#pragma unroll
+        for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { mk = k > mk ? k : mk; });
+        mk = block_max_u64<kCW>(mk, tmp);
+        const float s = scaled_of(bf16_of_key(kloc), a.temperature);
+        if (kloc && fabsf(s) < 0x1p30f && s >= scaled_of(bf16_of_key((uint32_t)mk), a.temperature) - 50.0f) {
+            each_top([&](uint32_t k, int64_t i, uint32_t, uint32_t r) {
+                if (k > kloc || r < room) return;
+                float val;
+                const uint64_t key = draw_key(s, a.seed, m, i, &val);
+                best = key > best ? key : best;
+            });
+            best = block_max_u64<kCW>(best, tmp);
+        }
+    }
+    if (tid == 0) {
+        a.info[m * a.P + p] = ((uint64_t)left << 32) | (kloc << 16) | (over + ties - left);
+        if (left) a.tie[m * a.P + p] = best;
+    }
 }
 
 // Exclusive prefix over the block of one count per thread; *total the sum.
@@ -993,19 +1057,22 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     __shared__ uint32_t tmp32[kWaves];
     __shared__ uint64_t sel[2];
     __shared__ uint32_t selk[2];
-    __shared__ uint32_t off[kThreads + 1];
-    // ---- the chunks' lists, one after the other (P <= kThreads) ----
+    __shared__ uint32_t off[kThreads];
+    __shared__ uint32_t upre[kThreads];                // unlisted ties at the k-th key in the chunks before
+    __shared__ uint32_t cut;                           // a chunk has unlisted ties
+    __shared__ uint32_t part[3];                       // 1 + the chunk kept in part, its listed ties, its kept ones
+    // ---- the chunks' lists, one after the other (P <= kThreads; at most
+    // P cap <= kListCap entries) ----
     uint32_t L;
-    const uint32_t nc = tid < a.P ? a.count[m * a.P + tid] : 0u;
-    off[tid] = block_prefix(nc, tmp32, &L);
+    const uint64_t info = tid < a.P ? a.info[m * a.P + tid] : 0u;
+    if (tid == 0) cut = part[0] = 0;
+    off[tid] = block_prefix((uint32_t)info & 0xffffu, tmp32, &L);
+    if (info >> 32) cut = 1;
 #pragma unroll
     for (int i = 0; i < kDigitBins / kThreads; ++i) hist[i * kThreads + tid] = 0;
     __syncthreads();
-    if (L > (uint32_t)kListCap) {                      // block-uniform
-        const int64_t S = ((a.N + kWaves * 512 - 1) / (kWaves * 512)) * 512;
-        sample_row<8>(m, a.logits, a.N, S, a.temperature, a.top_k, a.top_p, a.seed, a.idx, nullptr);
-        return;
-    }
+    const uint32_t klast = (uint32_t)info >> 16, left = (uint32_t)(info >> 32);   // of chunk tid
+    if (left) atomicAdd(&hist[klast >> kDigitShift], left);
     uint64_t mk = 0;
     for (int p = wave; p < a.P; p += kWaves) {
         const uint64_t* src = a.list + (m * a.P + p) * a.cap;
@@ -1019,12 +1086,13 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
         }
     }
     const uint32_t kmax = (uint32_t)block_max_u64<kWaves>(mk, tmp);   // its barriers also complete hist and cand
-    // ---- the k-th largest key (the lists hold at least top_k elements) ----
+    // ---- the k-th largest key (listed and counted, at least top_k elements) ----
     if (wave == 0) select_top_bin<kDigitBins / 64>(hist, (uint32_t)a.top_k, selk);
     __syncthreads();
     const uint32_t hb = selk[0], above = selk[1];
     if (tid < 256) hist[tid] = 0;
     __syncthreads();
+    if (left && (klast >> kDigitShift) == hb) atomicAdd(&hist[klast & ((1u << kDigitShift) - 1u)], left);
     for (uint32_t i = tid; i < L; i += kThreads) {
         const uint32_t k = (uint32_t)cand[i] & 0xffffu;
         if ((k >> kDigitShift) == hb) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], 1u);
@@ -1037,6 +1105,12 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     if (kmax < kmin) {                                 // nothing but NaN
         if (tid == 0) a.idx[m] = 0u;
         return;
+    }
+    // ---- ties at the k-th key that their chunks did not list ----
+    uint32_t u = 0, U = 0;                             // of chunk tid; of the row
+    if (cut) {                                         // block-uniform
+        u = klast == kmin ? left : 0u;
+        upre[tid] = block_prefix(u, tmp32, &U);
     }
     // ---- the elements from there on, in index order, to the front of cand ----
     constexpr int kPer = kListCap / kThreads;
@@ -1061,9 +1135,14 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     int64_t tie_keep = -1;                             // -1: every element equal to kstar is kept
     const float smax = scaled_of(bf16_of_key(kmax), T);
     if (a.use_p && mass_defined(smax)) {
+        const uint64_t fu = U ? U * fixed_mass(scaled_of(bf16_of_key(kmin), T), smax) : 0u;
         if (tid < 256) mass[tid] = 0;
         __syncthreads();
         uint64_t z = 0;
+        if (fu && tid == 0) {
+            z = fu;
+            atomicAdd(&mass[kmin >> 8], (unsigned long long)fu);
+        }
         for (uint32_t i = tid; i < F; i += kThreads) {
             const uint32_t k = (uint32_t)cand[i] & 0xffffu;
             const uint64_t f = fixed_mass(scaled_of(bf16_of_key(k), T), smax);
@@ -1079,6 +1158,7 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
         __syncthreads();
         if (tid < 256) mass[tid] = 0;
         __syncthreads();
+        if (fu && tid == 0 && (kmin >> 8) == hbp) atomicAdd(&mass[kmin & 0xffu], (unsigned long long)fu);
         for (uint32_t i = tid; i < F; i += kThreads) {
             const uint32_t k = (uint32_t)cand[i] & 0xffffu;
             if ((k >> 8) != hbp) continue;
@@ -1095,16 +1175,19 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
     }
     // ---- Gumbel-max over the kept elements, each thread a run of them ----
     const uint32_t per = (F + kThreads - 1) / kThreads, b = tid * per, e1 = b + per < F ? b + per : F;
+    const uint32_t C = (uint32_t)a.C;
+    // the top-p mask ends among the ties at the k-th key: ranks count the unlisted ones
+    const bool ranked = U && tie_keep >= 0 && kstar == kmin;
     uint32_t ties = 0, all;
     for (uint32_t i = b; i < e1; ++i) ties += ((uint32_t)cand[i] & 0xffffu) == kstar ? 1u : 0u;
-    int64_t below = (int64_t)block_prefix(ties, tmp32, &all);  // ties at kstar before this run
+    int64_t below = (int64_t)block_prefix(ties, tmp32, &all);  // listed ties at kstar before this run
     uint64_t best = 0;
     for (uint32_t i = b; i < e1; ++i) {
         const uint64_t v = cand[i];
         const uint32_t k = (uint32_t)v & 0xffffu;
         bool keep = k <= kstar;
         if (tie_keep >= 0 && k == kstar) {
-            keep = keep && below < tie_keep;
+            keep = keep && below + (ranked ? (int64_t)upre[(uint32_t)(v >> 16) / C] : 0) < tie_keep;
             ++below;
         }
         if (!keep) continue;
@@ -1112,25 +1195,77 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
         const uint64_t key = draw_key(scaled_of(bf16_of_key(k), T), a.seed, m, (int64_t)(v >> 16), &val);
         best = key > best ? key : best;
     }
+    if (U) {                                           // block-uniform, as ranked is
+        int64_t kept = u;                              // of chunk tid's unlisted ties
+        if (ranked) {
+            // their ranks follow the ties of the chunks before and the chunk's listed ones
+            hist[tid] = 0;
+            __syncthreads();
+            for (uint32_t i = tid; i < F; i += kThreads) {
+                const uint64_t v = cand[i];
+                if (((uint32_t)v & 0xffffu) == kstar) atomicAdd(&hist[(uint32_t)(v >> 16) / C], 1u);
+            }
+            __syncthreads();
+            const uint32_t listed = hist[tid];
+            const int64_t rest = tie_keep - (int64_t)block_prefix(listed, tmp32, &all) - listed - upre[tid];
+            kept = rest < 0 ? 0 : rest < kept ? rest : kept;
+            if (kept > 0 && kept < (int64_t)u) {       // one chunk at most
+                part[0] = tid + 1;
+                part[1] = listed;
+                part[2] = (uint32_t)kept;
+            }
+            __syncthreads();
+        }
+        if (u && kept == (int64_t)u) {
+            const uint64_t key = a.tie[m * a.P + tid];
+            best = key > best ? key : best;
+        }
+        if (part[0]) {                                 // block-uniform; its unlisted ties again
+            static_assert(kListSteps * kStep == kThreads * 8, "a chunk in one load per thread");
+            const int64_t beg = (int64_t)(part[0] - 1) * a.C, end = beg + a.C < a.N ? beg + a.C : a.N;
+            const int64_t i0 = beg + tid * 8;
+            uint4 q = make_uint4(0, 0, 0, 0);
+            const bool ok = i0 < end;
+            if (ok) q = *reinterpret_cast<const uint4*>(a.logits + m * a.N + i0);
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+            uint32_t c = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                c += ok && bf16_order_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu) == kstar ? 1u : 0u;
+            uint32_t r = block_prefix(c, tmp32, &all);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (!ok || bf16_order_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu) != kstar) continue;
+                if (r >= part[1] && r < part[1] + part[2]) {
+                    float val;
+                    const uint64_t key = draw_key(scaled_of(bf16_of_key(kstar), T), a.seed, m, i0 + e, &val);
+                    best = key > best ? key : best;
+                }
+                ++r;
+            }
+        }
+    }
     best = block_max_u64<kWaves>(best, tmp);
     if (tid == 0) a.idx[m] = best ? argmax_key_index(best) : 0u;
 }
 
-// Chunks of the list path: the chain's, made larger until top_k (and some
-// ties) of every chunk fit the LDS list; false if they do not.
-inline bool list_shape(int64_t M, int64_t N, int top_k, int* P, int64_t* C) {
-    chunk_shape(M, N, P, C);
-    while (*C <= kListSteps * kStep) {
-        *P = (int)((N + *C - 1) / *C);
-        if (*P <= kThreads && (int64_t)*P * (top_k + 16) <= kListCap) return true;
-        *C *= 2;
+// Chunks and list lengths of the list path: the chain's chunks, made larger
+// until top_k (and some ties) of every chunk fit the LDS list; false if they
+// do not.
+inline bool list_shape(int64_t M, int64_t N, ListArgs* a) {
+    chunk_shape(M, N, &a->P, &a->C);
+    for (; a->C <= kListSteps * kStep; a->C *= 2) {
+        a->P = (int)((N + a->C - 1) / a->C);
+        if (a->P > kThreads) continue;
+        const int64_t want = (int64_t)a->top_k + kListTies;
+        a->cap = (int)(want < a->C ? want : a->C);
+        if ((int64_t)a->P * a->cap <= kListCap) return true;
     }
     return false;
 }
-// Workspace: a count per chunk (at most kThreads), and 2 kListCap entries per
-// row, shared evenly by its chunks (at least twice top_k + 16 each).
+// Workspace: two words per chunk (at most kThreads), and kListCap entries per row.
 inline size_t list_bytes(int64_t M) {
-    return align256((size_t)M * kThreads * 4) + (size_t)M * 2 * kListCap * 8;
+    return 2 * align256((size_t)M * kThreads * 8) + (size_t)M * kListCap * 8;
 }
 
 // Workspace carve-up of the chunked path; returns the bytes needed.
@@ -1219,19 +1354,20 @@ extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, flo
         // stages and as fast or faster (one row 19.7 us at every top_k, lists
         // 20.7 / 22.0 at 20 / 50; 4 rows 24.6, lists 21.1 to 27.3).
         const bool lists = a.use_k && !keep && (a.use_p || M * a.P > smp::kListMinChunks);
-        if (lists && smp::list_shape(M, N, top_k, &l.P, &l.C)) {
+        l.top_k = top_k;
+        if (lists && smp::list_shape(M, N, &l)) {
+            char* base = static_cast<char*>(workspace);
+            const size_t words = smp::align256((size_t)M * l.P * 8);
             l.logits = logits;
             l.N = N;
             l.temperature = temperature;
-            l.top_k = top_k;
             l.top_p = top_p;
             l.seed = seed;
             l.use_p = a.use_p;
             l.idx = idx;
-            l.count = static_cast<uint32_t*>(workspace);
-            l.list = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + smp::align256((size_t)M * smp::kThreads * 4));
-            const int64_t cap = 2 * smp::kListCap / l.P;
-            l.cap = (int)(cap < l.C ? cap : l.C);
+            l.info = reinterpret_cast<uint64_t*>(base);
+            l.tie = reinterpret_cast<uint64_t*>(base + words);
+            l.list = reinterpret_cast<uint64_t*>(base + 2 * words);
             hipLaunchKernelGGL(smp::topk_list_kernel, dim3((unsigned)l.P, (unsigned)M), dim3(smp::kCT), 0, st, l);
             hipLaunchKernelGGL(smp::list_draw_kernel, dim3((unsigned)M), dim3(smp::kThreads), 0, st, l);
             return launch_status(what);

@@ -224,7 +224,7 @@ def test_infinite_largest_value(mq4, dev, chunked):
 @pytest.mark.parametrize("M,V", [(1, 8192), (1, 8200), (3, 10248), (1, 151936), (4, 248320), (32, 65536), (128, 8192)])
 def test_candidate_lists_agree_with_single_workgroup(mq4, dev, M, V):
     """Top-k without a keep mask on candidate lists against the one-workgroup
-    path, token for token: odd last chunks, ties (lists that overflow, rows of
+    path, token for token: odd last chunks, ties (more than a list holds, rows of
     one value), infinities, NaN, a row of NaN, the lowest finite value, top_k
     from 1 past a chunk's size (the chain), with and without top-p."""
     rng = np.random.default_rng(300 + M + V)
@@ -252,3 +252,88 @@ def test_candidate_lists_agree_with_single_workgroup(mq4, dev, M, V):
             assert rc == 0, L.mq4_last_error()
             got.append(idx.cpu().numpy())
         assert np.array_equal(got[0], got[1]), (t, k, p, np.nonzero(got[0] != got[1])[0][:8])
+
+
+def masked_rows(kind, M, V, seed):
+    """Decoder logits with a masked or constant stretch."""
+    rng = np.random.default_rng(seed)
+    bits = gen_logits(rng, M, V, "normal")
+    i = np.arange(V)
+    if kind == "half":                                   # more kept than any top_k, half the row masked
+        bits[:, : V // 2] = 0xff80
+    elif kind == "half_lowest":
+        bits[:, : V // 2] = 0xff7f
+    elif kind == "grammar":                              # 200 allowed
+        bits[:, i % (V // 200) != 0] = 0xff80
+    elif kind == "grammar_few":                          # fewer allowed than top_k: the k-th key is the mask
+        bits[:, i % (V // 20) != 0] = 0xff80
+    elif kind == "few_finite_mask":
+        bits[:, i % (V // 20) != 0] = 0xc61c             # about -1e4
+    elif kind == "few_near":                             # the masked value keeps a mass and can be drawn
+        bits[:, i % (V // 20) != 0] = 0xc000
+    elif kind == "padding":
+        bits[:, V * 4 // 5 :] = 0
+    elif kind == "constant":
+        bits[:] = 0x3f80
+    elif kind == "none":
+        bits[:] = 0xff80
+    elif kind == "nan":
+        bits[:, V // 3 :] = 0x7fc0
+    elif kind == "grid":                                 # a few values throughout
+        bits[:] = gen_logits(rng, M, V, "ties")
+    return bits
+
+
+@pytest.mark.parametrize("M,V", [(1, 8192), (1, 16392), (2, 248320), (6, 248320), (9, 151944), (32, 65536)])
+def test_masked_rows_agree_with_single_workgroup(mq4, dev, M, V):
+    """Rows whose chunks tie at their own k-th key beyond what a candidate list
+    holds, with the row's k-th key above those ties or equal to them, and a
+    top-p mask that ends above, at and inside the ties: the one-workgroup
+    path's tokens."""
+    L = mq4.lib()
+    n = L.mq4_sample_workspace_size(M, V)
+    ws = torch.full((n,), 0xAB, dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    for kind in ("half", "half_lowest", "grammar", "grammar_few", "few_finite_mask", "few_near", "padding", "constant",
+                 "none", "nan", "grid"):
+        x = to_dev(masked_rows(kind, M, V, 900 + M), dev)
+        for t, k, p in [(0.7, 50, 0.9), (1.0, 200, 0.5), (1.0, 50, 0.003), (0.9, 17, 0.9999), (1.0, 1, 0.37), (0.8, 100, 1.0),
+                        (1.3, 300, 0.02)]:
+            print(f"masked {kind} M={M} V={V} t={t} k={k} p={p}", flush=True)
+            got = []
+            for w, b in ((ws.data_ptr(), n), (None, 0)):
+                idx = torch.full((M,), -7, dtype=torch.int32, device=dev)
+                rc = L.mq4_sample_bf16(x.data_ptr(), M, V, t, k, p, 4321 + k, idx.data_ptr(), None, w, b, stream)
+                assert rc == 0, L.mq4_last_error()
+                got.append(idx.cpu().numpy())
+            assert np.array_equal(got[0], got[1]), (kind, t, k, p, np.nonzero(got[0] != got[1])[0][:8])
+
+
+@pytest.mark.parametrize("kind", ["half", "grammar", "grammar_few", "few_near", "constant"])
+def test_masked_rows_take_no_longer(mq4, dev, kind):
+    """A masked or constant row keeps the candidate lists' time (one workgroup
+    over the whole row takes 12 to 50 times as long): within three times an
+    ordinary row's, far outside the spread of a box."""
+    L = mq4.lib()
+    V = 248320
+    n = L.mq4_sample_workspace_size(1, V)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    idx = torch.empty(1, dtype=torch.int32, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def best_us(x):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(5):
+            e0.record()
+            for _ in range(30):
+                assert L.mq4_sample_bf16(x.data_ptr(), 1, V, 0.7, 50, 0.9, 5, idx.data_ptr(), None, ws.data_ptr(), n,
+                                         stream) == 0
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 1000 / 30)
+        return best
+
+    print(f"masked row time {kind}", flush=True)
+    plain, masked = (best_us(to_dev(masked_rows(q, 1, V, 3), dev)) for q in ("plain", kind))
+    assert masked < 3 * plain, (plain, masked)
