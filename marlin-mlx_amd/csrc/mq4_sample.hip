@@ -840,9 +840,9 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // stages of 3 to 13 us).
 //   topk_list   each chunk selects its own top_k largest keys in LDS, and
 //               writes them with their indices in index order.  The ties of
-//               the last one are all listed if they fit into top_k +
-//               kListTies entries; else the first kListTies, and of the rest
-//               the chunk writes their number and their best draw.  The row's
+//               the last one are all listed if they fit the list; else the
+//               first kListTies, and of the rest the chunk writes their number
+//               and their best draw.  The row's
 //               k-th largest key is at least every chunk's, so it follows
 //               from the lists and these numbers, and every kept element is
 //               on a list or is one of the counted ties.
@@ -863,7 +863,7 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // 676 and 1234, on the chain 39.0, 39.9, 43.2 and 46.9.
 constexpr int kListCap = 15360;             // candidates of a row in LDS (120 KB)
 constexpr int64_t kListMinChunks = 512;     // without top-p: chunks of a call above which lists pay
-constexpr int kListTies = 16;               // list entries of a chunk beyond top_k
+constexpr int kListTies = 16;               // list entries of a chunk beyond top_k, at least
 constexpr int kListSteps = 4;               // steps of a chunk held in registers: C <= 4 kStep
 // Radix digits of the lists' selections: 11 bits, then 5.  Logits share few
 // sign and exponent bits, and LDS atomics of a wave to one bin go one by one:
@@ -972,47 +972,54 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
         total += tot;
     }
     const uint32_t ties = total >> 16;
-    // All of the ties are listed if they fit, else the first few.
-    const uint32_t fit = (uint32_t)a.cap - over;
-    const uint32_t room = ties <= fit ? fit : (uint32_t)kListTies;   // then cap = top_k + kListTies
-    const uint32_t left = ties > room ? ties - room : 0u;       // block-uniform
     uint64_t* list = a.list + (m * a.P + p) * a.cap;
-    // f(key, element, keys above kloc before it, ties before it) over the
-    // logits from kloc up, in this thread's order
-    auto each_top = [&](auto&& f) {
+    auto index = [&](int t, int e) { return beg + (int64_t)t * kStep + tid * 8 + e; };
+    uint32_t left = 0;                                 // ties not listed
+    uint64_t best = 0;                                 // the best draw of those
+    if (over + ties <= (uint32_t)a.cap) {              // block-uniform
 #pragma unroll
         for (int t = 0; t < kListSteps; ++t) {
-            uint32_t at = cnt[t];
+            uint32_t at = (cnt[t] & 0xffffu) + (cnt[t] >> 16);
             each(t, [&](uint32_t k, int e) {
-                if (k < kloc) return;
-                f(k, beg + (int64_t)t * kStep + tid * 8 + e, at & 0xffffu, at >> 16);
-                at += k > kloc ? 1u : 0x10000u;
+                if (k >= kloc) list[at++] = ((uint64_t)index(t, e) << 16) | k;
             });
         }
-    };
-    each_top([&](uint32_t k, int64_t i, uint32_t g, uint32_t r) {
-        if (k > kloc || r < room) list[g + (r < room ? r : room)] = ((uint64_t)i << 16) | k;
-    });
-    uint64_t best = 0;
-    if (left) {
-        // The best draw of the ties not listed.  Not needed for NaN (never
-        // kept); where the Gumbel noise (below 2^5) is lost in the value, as
-        // the listed ties come first then; nor for a value 50 below the
-        // chunk's largest, when it cannot win: the largest element that top-p
-        // keeps has a mass of at least 2^-41 of the largest one's, so its
-        // value is within 28.5 of that, and noise lies in (-3, kGumbelMax).
+    } else {
+        // Longer than the list (so cap < C, and cap >= top_k + kListTies):
+        // the first kListTies ties.
+        constexpr uint32_t room = kListTies;
+        left = ties - room;
         uint64_t mk = 0;
 #pragma unroll
-        for (int t = 0; t < kListSteps; ++t) each(t, [&](uint32_t k, int) { mk = k > mk ? k : mk; });
+        for (int t = 0; t < kListSteps; ++t) {
+            uint32_t g = cnt[t] & 0xffffu, r = cnt[t] >> 16;
+            each(t, [&](uint32_t k, int e) {
+                mk = k > mk ? k : mk;
+                if (k < kloc) return;
+                if (k > kloc || r < room) list[g + (r < room ? r : room)] = ((uint64_t)index(t, e) << 16) | k;
+                g += k > kloc ? 1u : 0u;
+                r += k > kloc ? 0u : 1u;
+            });
+        }
+        // The best draw of the others.  Not needed for NaN (never kept); where
+        // the Gumbel noise (below 2^5) is lost in the value, as the listed
+        // ties come first then; nor for a value 50 below the chunk's largest,
+        // when it cannot win: the largest element that top-p keeps has a mass
+        // of at least 2^-41 of the largest one's, so its value is within 28.5
+        // of that, and noise lies in (-3, kGumbelMax).
         mk = block_max_u64<kCW>(mk, tmp);
         const float s = scaled_of(bf16_of_key(kloc), a.temperature);
         if (kloc && fabsf(s) < 0x1p30f && s >= scaled_of(bf16_of_key((uint32_t)mk), a.temperature) - 50.0f) {
-            each_top([&](uint32_t k, int64_t i, uint32_t, uint32_t r) {
-                if (k > kloc || r < room) return;
-                float val;
-                const uint64_t key = draw_key(s, a.seed, m, i, &val);
-                best = key > best ? key : best;
-            });
+#pragma unroll
+            for (int t = 0; t < kListSteps; ++t) {
+                uint32_t r = cnt[t] >> 16;
+                each(t, [&](uint32_t k, int e) {
+                    if (k != kloc || r++ < room) return;
+                    float val;
+                    const uint64_t key = draw_key(s, a.seed, m, index(t, e), &val);
+                    best = key > best ? key : best;
+                });
+            }
             best = block_max_u64<kCW>(best, tmp);
         }
     }
@@ -1250,22 +1257,32 @@ __global__ __launch_bounds__(kThreads) void list_draw_kernel(ListArgs a) {
 }
 
 // Chunks and list lengths of the list path: the chain's chunks, made larger
-// until top_k (and some ties) of every chunk fit the LDS list; false if they
-// do not.
-inline bool list_shape(int64_t M, int64_t N, ListArgs* a) {
+// until top_k and kListTies ties of every chunk fit its share of the LDS list
+// and of a workspace of `bytes` (two words per chunk, then the lists); false
+// if they do not.
+inline bool list_shape(int64_t M, int64_t N, size_t bytes, ListArgs* a) {
     chunk_shape(M, N, &a->P, &a->C);
     for (; a->C <= kListSteps * kStep; a->C *= 2) {
         a->P = (int)((N + a->C - 1) / a->C);
-        if (a->P > kThreads) continue;
-        const int64_t want = (int64_t)a->top_k + kListTies;
-        a->cap = (int)(want < a->C ? want : a->C);
-        if ((int64_t)a->P * a->cap <= kListCap) return true;
+        const size_t chunks = (size_t)M * a->P, words = 2 * align256(chunks * 8);
+        if (a->P > kThreads || bytes < words) continue;
+        const int64_t want = (int64_t)a->top_k + kListTies, fit = (int64_t)((bytes - words) / (chunks * 8));
+        int64_t cap = kListCap / a->P < a->C ? kListCap / a->P : a->C;
+        cap = cap < fit ? cap : fit;
+        a->cap = (int)cap;
+        if (cap >= (want < a->C ? want : a->C)) return true;
     }
     return false;
 }
-// Workspace: two words per chunk (at most kThreads), and kListCap entries per row.
-inline size_t list_bytes(int64_t M) {
-    return 2 * align256((size_t)M * kThreads * 8) + (size_t)M * kListCap * 8;
+// The most that list_shape uses at any top_k; 0 where it holds for none.
+// (Above the chain's partials, 7184 bytes per chunk, only for few chunks per
+// row, where lists of more than 880 keys fit the LDS.)
+inline size_t list_bytes(int64_t M, int64_t N) {
+    ListArgs a{};
+    a.top_k = 1;
+    if (!list_shape(M, N, ~(size_t)0, &a)) return 0;
+    const int64_t whole = (N + kListSteps * kStep - 1) / (kListSteps * kStep) * (kListSteps * kStep);
+    return 2 * align256((size_t)M * a.P * 8) + (size_t)(M * (whole < kListCap ? whole : kListCap)) * 8;
 }
 
 // Workspace carve-up of the chunked path; returns the bytes needed.
@@ -1304,12 +1321,17 @@ inline size_t chunk_layout(int64_t M, int P, char* base, ChunkArgs* a) {
 
 using namespace mq4;
 
-extern "C" size_t mq4_sample_workspace_size(int64_t M, int64_t N) {
+// Bytes of the chain's partials; 0 where rows are not chunked.
+static size_t chain_bytes(int64_t M, int64_t N) {
     if (M <= 0 || N <= 0 || !smp::chunk_eligible(M, N)) return 0;
     int P;
     int64_t C;
     smp::chunk_shape(M, N, &P, &C);
-    const size_t chain = smp::chunk_layout(M, P, nullptr, nullptr), lists = smp::list_bytes(M);
+    return smp::chunk_layout(M, P, nullptr, nullptr);
+}
+
+extern "C" size_t mq4_sample_workspace_size(int64_t M, int64_t N) {
+    const size_t chain = chain_bytes(M, N), lists = chain ? smp::list_bytes(M, N) : 0;
     return chain > lists ? chain : lists;
 }
 
@@ -1328,7 +1350,7 @@ extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, flo
         return fail(MQ4_ERR_INVALID_ARG, "%s: temperature and top_p must not be NaN", what);
     const bool vec8 = N % 8 == 0 && aligned(logits, 16) && (!keep || aligned(keep, 8));
     const hipStream_t st = as_stream(stream);
-    const size_t need = mq4_sample_workspace_size(M, N);
+    const size_t need = chain_bytes(M, N);             // the lists take what they fit
     if (workspace && need && vec8) {
         if (workspace_bytes < need || !aligned(workspace, 256))
             return fail(MQ4_ERR_WORKSPACE, "%s: workspace of %zu bytes (256-byte aligned) needed, got %zu", what,
@@ -1355,7 +1377,7 @@ extern "C" int mq4_sample_bf16(const uint16_t* logits, int64_t M, int64_t N, flo
         // 20.7 / 22.0 at 20 / 50; 4 rows 24.6, lists 21.1 to 27.3).
         const bool lists = a.use_k && !keep && (a.use_p || M * a.P > smp::kListMinChunks);
         l.top_k = top_k;
-        if (lists && smp::list_shape(M, N, &l)) {
+        if (lists && smp::list_shape(M, N, workspace_bytes, &l)) {
             char* base = static_cast<char*>(workspace);
             const size_t words = smp::align256((size_t)M * l.P * 8);
             l.logits = logits;

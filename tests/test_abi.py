@@ -158,6 +158,22 @@ def test_sample_validation(mq4):
     assert L.mq4_sample_bf16(*ws_args, fake(A16 + 8), need, S) == WORKSPACE
 
 
+@pytest.mark.parametrize("M,N,lists", [(1, 8192, 8192), (1, 248320, 0), (8, 8200, 15360), (33, 151944, 0),
+                                       (34, 248320, 0), (64, 65536, 15360), (128, 248320, 0)])
+def test_sample_workspace_size(mq4, M, N, lists):
+    """mq4_sample_workspace_size: the chunk chain's partial results (per chunk
+    two words, three histograms of 256 counts and two of 256 masses; 40 bytes
+    per row), or the candidate lists (two words per chunk, at most 15360
+    entries per row) where they can be longer; each section 256-byte aligned.
+    Shapes that no list serves ask for the chain's alone."""
+    up = lambda v: (v + 255) // 256 * 256
+    steps = -(-N // 2048)
+    C = -(-steps // max(1, 1024 // M)) * 2048
+    mp = M * -(-N // C)
+    chain = 2 * up(8 * mp) + 3 * up(1024 * mp) + 2 * up(2048 * mp) + up(40 * M)
+    assert mq4.lib().mq4_sample_workspace_size(M, N) == max(chain, 2 * up(8 * mp) + 8 * M * lists if lists else 0)
+
+
 class _Layer(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in (
         "norm_weight", "gate_wq", "gate_scales", "gate_biases", "up_wq", "up_scales", "up_biases",

@@ -297,8 +297,8 @@ def test_masked_rows_agree_with_single_workgroup(mq4, dev, M, V):
     for kind in ("half", "half_lowest", "grammar", "grammar_few", "few_finite_mask", "few_near", "padding", "constant",
                  "none", "nan", "grid"):
         x = to_dev(masked_rows(kind, M, V, 900 + M), dev)
-        for t, k, p in [(0.7, 50, 0.9), (1.0, 200, 0.5), (1.0, 50, 0.003), (0.9, 17, 0.9999), (1.0, 1, 0.37), (0.8, 100, 1.0),
-                        (1.3, 300, 0.02)]:
+        for t, k, p in [(0.7, 50, 0.9), (1.0, 200, 0.5), (1.0, 50, 0.003), (0.9, 17, 0.9999), (1.0, 1, 0.37),
+                        (0.8, 100, 1.0), (1.3, 300, 0.02)]:
             print(f"masked {kind} M={M} V={V} t={t} k={k} p={p}", flush=True)
             got = []
             for w, b in ((ws.data_ptr(), n), (None, 0)):
@@ -307,6 +307,38 @@ def test_masked_rows_agree_with_single_workgroup(mq4, dev, M, V):
                 assert rc == 0, L.mq4_last_error()
                 got.append(idx.cpu().numpy())
             assert np.array_equal(got[0], got[1]), (kind, t, k, p, np.nonzero(got[0] != got[1])[0][:8])
+
+
+def chain_bytes(M, V):
+    """Bytes of the chunk chain's partial results."""
+    up = lambda v: (v + 255) // 256 * 256
+    C = -(-(-(-V // 2048)) // max(1, 1024 // M)) * 2048
+    mp = M * -(-V // C)
+    return 2 * up(8 * mp) + 3 * up(1024 * mp) + 2 * up(2048 * mp) + up(40 * M)
+
+
+@pytest.mark.parametrize("M,V", [(1, 8192), (3, 16392), (32, 248320), (34, 248320), (64, 65536), (128, 8192), (128, 65536)])
+def test_lists_stay_in_the_workspace(mq4, dev, M, V):
+    """top_k up to the largest that the lists take, and past it, in a workspace
+    of the stated size and in one of the chain's alone (enough for every call;
+    longer lists are not used then): accepted, nothing written behind it, and
+    the one-workgroup path's tokens."""
+    L = mq4.lib()
+    sizes = (L.mq4_sample_workspace_size(M, V), chain_bytes(M, V))
+    assert sizes[0] >= sizes[1]
+    x = to_dev(gen_logits(np.random.default_rng(M + V), M, V, "normal"), dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    for k in (50, 464, 880, 881, 1000, 1904, 3824, 7000):
+        print(f"list workspace M={M} V={V} k={k}", flush=True)
+        want = torch.full((M,), -7, dtype=torch.int32, device=dev)
+        assert L.mq4_sample_bf16(x.data_ptr(), M, V, 0.9, k, 0.8, 11, want.data_ptr(), None, None, 0, stream) == 0
+        for n in sizes:
+            ws = torch.full((n + 65536,), 0x5A, dtype=torch.uint8, device=dev)
+            idx = torch.full((M,), -7, dtype=torch.int32, device=dev)
+            rc = L.mq4_sample_bf16(x.data_ptr(), M, V, 0.9, k, 0.8, 11, idx.data_ptr(), None, ws.data_ptr(), n, stream)
+            assert rc == 0, L.mq4_last_error()
+            assert torch.equal(idx, want), (k, n)
+            assert (ws[n:] == 0x5A).all(), (k, n)
 
 
 @pytest.mark.parametrize("kind", ["half", "grammar", "grammar_few", "few_near", "constant"])
