@@ -189,7 +189,10 @@ int mq4_rmsnorm_gate_up_silu(const uint16_t* x, int64_t M, int64_t K,
  * N) bytes, 256-byte aligned, no initialisation; calls that overlap in time
  * need separate workspaces.  y may equal x (in place).
  * mq4_mlp_workspace_size(M, K, N) is enough for every call of at most M rows
- * with the same K and N: it never shrinks as M grows. */
+ * with the same K and N: it never shrinks as M grows.  (A workspace that is
+ * smaller than a call's own layout by K parts of the down product is accepted
+ * down to 4, 2 or 1 of them; the call then runs on as many as it holds, which
+ * is slower and sums in another order.) */
 size_t mq4_mlp_workspace_size(int64_t M, int64_t K, int64_t N);
 int mq4_mlp_residual(const uint16_t* x, int64_t M, int64_t K,
                      const uint16_t* norm_weight, float eps,

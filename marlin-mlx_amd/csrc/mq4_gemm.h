@@ -75,8 +75,9 @@ struct Gemm16Args {
 int launch_q4_gemm16(const Gemm16Args& a, int epi, hipStream_t st);
 
 // K parts of the fp16-weight GEMM_RESIDUAL product of this shape (K % 512 ==
-// 0); changes with M at multiples of 64 only, and past 128 rows never grows.
-int gemm16_parts(int64_t M, int64_t N, int64_t K);
+// 0), at most `most`; changes with M at multiples of 64 only, and past 128
+// rows never grows.
+int gemm16_parts(int64_t M, int64_t N, int64_t K, int most = 6);
 
 // xp = fp16(x / xscale[m]) (norm_w null) or fp16(bf16(x * rsqrt(mean(x^2) +
 // eps) * (1 + norm_w)) / xscale[m]) in the operand order, by k group (the bits of

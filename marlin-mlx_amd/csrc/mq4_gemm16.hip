@@ -882,16 +882,16 @@ Tile tile_for(int64_t M, int64_t N, int64_t K, int epi) {
 
 }  // namespace g16
 
-// The most K parts (whole eight-group blocks per part and team) whose blocks
-// stay within one per CU.
-int gemm16_parts(int64_t M, int64_t N, int64_t K) {
+// The most K parts, up to `most` (whole eight-group blocks per part and team),
+// whose blocks stay within one per CU.
+int gemm16_parts(int64_t M, int64_t N, int64_t K, int most) {
     const g16::Tile t = g16::tile_for(M, N, K, GEMM_RESIDUAL);
     const int64_t r = t == g16::T64x128 ? 64 : t == g16::T256x256 ? 256 : 128;
     const int64_t c = t == g16::T64x128 || t == g16::T128x128 ? 128 : 256;
     const int64_t blocks = ((M + r - 1) / r) * ((N + c - 1) / c), teams = t == g16::T64x128 ? 2 : 1;
     int S = 1;
     for (int s : {2, 3, 4, 6})
-        if ((K / 512) % (s * teams) == 0 && blocks * s <= (int64_t)num_cus()) S = s;
+        if (s <= most && (K / 512) % (s * teams) == 0 && blocks * s <= (int64_t)num_cus()) S = s;
     return S;
 }
 

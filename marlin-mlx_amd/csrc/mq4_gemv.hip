@@ -772,9 +772,19 @@ struct MlpWs {
 
 // K parts of the fp16-weight down product ([M, N] . [K, N]^T); 0: N / 64 not
 // a multiple of 8 (no fp16 down product).
-static int mlp_down_parts(int64_t M, int64_t K, int64_t N) { return N % 512 != 0 ? 0 : gemm16_parts(M, K, N); }
+static int mlp_down_parts(int64_t M, int64_t K, int64_t N, int most = 6) {
+    return N % 512 != 0 ? 0 : gemm16_parts(M, K, N, most);
+}
+// The K parts that a workspace has to hold at least: of mlp_down_parts the
+// most of 1, 2 and 4 that divide K.  A call takes as many parts as its
+// workspace holds, so a size kept from when 4 was the limit stays enough.
+static int mlp_least_parts(int64_t M, int64_t K, int64_t N) {
+    const int S = mlp_down_parts(M, K, N);
+    return S >= 4 && N % 2048 == 0 ? 4 : S >= 2 && N % 1024 == 0 ? 2 : S >= 1 ? 1 : 0;
+}
 
-static MlpWs mlp_ws_layout(void* base, int64_t M, int64_t K, int64_t N) {
+// The layout with the down product in S K parts.
+static MlpWs mlp_ws_layout(void* base, int64_t M, int64_t K, int64_t N, int S) {
     MlpWs w;
     char* b = reinterpret_cast<char*>(base);
     size_t off = 0;
@@ -789,7 +799,6 @@ static MlpWs mlp_ws_layout(void* base, int64_t M, int64_t K, int64_t N) {
         w.xp = reinterpret_cast<uint16_t*>(take((size_t)M * K * 2));
         w.xs = reinterpret_cast<float*>(take((size_t)M * (K / 64) * 4));
         w.hs = reinterpret_cast<float*>(take((size_t)M * (N / 64) * 4));
-        const int S = mlp_down_parts(M, K, N);
         if (S > 1) w.kpart = reinterpret_cast<float*>(take((size_t)S * M * K * 4));
         w.silu = reinterpret_cast<uint16_t*>(take((size_t)SILU_LUT_N * 2));
     } else if (M >= kMfmaMinM) {
@@ -818,12 +827,13 @@ static bool mlp_paired_ok(int64_t M, int64_t K, int64_t N, const QMat& g, const 
 // and the row counts just below a drop (multiples of 64), up to M.
 extern "C" size_t mq4_mlp_workspace_size(int64_t M, int64_t K, int64_t N) {
     if (M <= 0 || K <= 0 || N <= 0) return 0;
-    size_t need = mlp_ws_layout(nullptr, M, K, N).bytes;
+    size_t need = 0;
     auto at = [&](int64_t m) {
         if (m < 1 || m > M) return;
-        const size_t b = mlp_ws_layout(nullptr, m, K, N).bytes;
+        const size_t b = mlp_ws_layout(nullptr, m, K, N, mlp_down_parts(m, K, N)).bytes;
         need = b > need ? b : need;
     };
+    at(M);
     at(kMfmaMinM - 1);
     at(kGemmMinM - 1);
     for (int64_t m = 64; m < M; m += 64) {
@@ -844,11 +854,14 @@ extern "C" int mq4_mlp_residual(const uint16_t* x, int64_t M, int64_t K, const u
     if (int rc = check_qmm_args(what, x, M, K, up_wq, up_scales, up_biases, N)) return rc;
     if (int rc = check_norm(what, norm_weight, eps)) return rc;
     if (!y || !aligned(y, 2)) return fail(MQ4_ERR_INVALID_ARG, "%s: y must be a 2-byte aligned pointer", what);
-    const size_t need = mlp_ws_layout(nullptr, M, K, N).bytes;
+    auto bytes = [&](int parts) { return mlp_ws_layout(nullptr, M, K, N, parts).bytes; };
+    const size_t need = bytes(mlp_least_parts(M, K, N));
     if (!workspace || workspace_bytes < need || !aligned(workspace, 256))
         return fail(MQ4_ERR_WORKSPACE, "%s: workspace needs %zu bytes, 256-byte aligned (got %zu)", what, need,
                     workspace_bytes);
-    const MlpWs w = mlp_ws_layout(workspace, M, K, N);
+    int parts = mlp_down_parts(M, K, N);
+    while (parts > 1 && bytes(parts) > workspace_bytes) parts = mlp_down_parts(M, K, N, parts - 1);
+    const MlpWs w = mlp_ws_layout(workspace, M, K, N, parts);
     if (int rc = check_qmm_args(what, w.h, M, N, down_wq, down_scales, down_biases, K)) return rc;
     const QMat G{gate_wq, gate_scales, gate_biases}, U{up_wq, up_scales, up_biases},
         D{down_wq, down_scales, down_biases};
@@ -868,7 +881,7 @@ extern "C" int mq4_mlp_residual(const uint16_t* x, int64_t M, int64_t K, const u
         if (a16(G) && a16(U)) {
             // K parts need an 8-byte aligned y (one part stores any 2-byte
             // aligned y element by element)
-            int parts = a16(D) ? mlp_down_parts(M, K, N) : 0;
+            if (!a16(D)) parts = 0;
             if (parts > 1 && !aligned(y, 8)) parts = 1;
             const bool down16 = parts > 0;
             if (launch_pair_rows16(x, (int)M, (int)K, norm_weight, eps, w.xp, w.xs, w.silu, st))

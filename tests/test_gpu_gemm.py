@@ -433,6 +433,40 @@ def test_mlp_residual_split_graph_replay(mq4, O, dev, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,parts", [(40, 2048, 6144, 4), (128, 2048, 6144, 4), (203, 2048, 6144, 4),
+                                         (600, 2048, 6144, 2), (200, 1024, 3072, 2), (256, 1024, 3072, 2)])
+def test_mlp_residual_smaller_workspace(mq4, O, dev, M, K, N, parts):
+    """A workspace for `parts` K parts of the down product, where the call
+    would run on more (6, 6, 6, 3, 3 or 6): accepted, nothing written behind
+    it, and the same product in another summation order (the fp32 sums differ
+    by about 1e-6 of the output's rms: bf16 results differ only at roundings).
+    One byte less is refused."""
+    up = lambda v: (v + 255) // 256 * 256
+    nb = (up(M * N * 2) + up(M * K * 2) + up(M * K // 64 * 4) + up(M * N // 64 * 4) + up(parts * M * K * 4) + 8192)
+    L = mq4.lib()
+    assert nb < L.mq4_mlp_workspace_size(M, K, N)
+    print(f"mlp_residual smaller workspace M={M} K={K} N={N}", flush=True)
+    ws_ = [make(mq4, O, *((N, K) if p < 2 else (K, N)), 1500 + p, dev)[0] for p in range(3)]
+    x = mq4.fill_normal_bf16((M, K), mq4.STREAM_PREFILL + 5, 0.0, 1.0, device=dev)
+    nw = mq4.fill_normal_bf16((K,), mq4.stream_id_layer_norm(5), 0.1, 0.02, device=dev)
+    want = mq4.mlp_residual(x, mq4.MLPWeights(*[mq4.QuantizedTensor(*d) for d in ws_]), nw, 1e-6)
+    ws = torch.full((nb + 4096,), 0x5A, dtype=torch.uint8, device=dev)
+    y = torch.empty_like(x)
+    w9 = [t.data_ptr() for d in ws_ for t in d]
+    call = lambda n: L.mq4_mlp_residual(x.data_ptr(), M, K, nw.data_ptr(), 1e-6, *w9, N, ws.data_ptr(), n,
+                                        y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert call(nb - 1) == -5                              # MQ4_ERR_WORKSPACE
+    assert call(nb) == 0, L.mq4_last_error()
+    torch.cuda.synchronize()
+    assert (ws[nb:] == 0x5A).all()
+    got, ref = to_host_u16(y), to_host_u16(want)
+    assert np.mean(got == ref) >= 0.99
+    d = (O.bf16_to_f32(got) - O.bf16_to_f32(ref)).astype(np.float64)
+    m = O.bf16_to_f32(ref).astype(np.float64) - O.bf16_to_f32(to_host_u16(x))
+    assert np.sqrt(np.mean(d * d) / np.mean(m * m)) <= 1e-3
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N", [(33, 2048, 6144), (64, 2048, 6144), (65, 2048, 6144), (128, 2048, 6144),
                                    (129, 2048, 6144), (192, 2048, 6144), (256, 2048, 6144), (257, 2048, 6144),
                                    (385, 2048, 6144), (513, 2048, 6144), (2049, 2048, 6144), (4097, 2048, 6144),
