@@ -87,11 +87,16 @@ __device__ __forceinline__ bf16x8_t weight_operand(uint32_t word) {
 }
 
 // weight_operand with the mask (SGPR) and exponent bits (VGPR) held by the
-// caller: one v_and_or_b32 per nibble pair plus a shift for pairs 1-3.
+// caller: one v_and_or_b32 per nibble pair plus a shift for pairs 1-3.  The
+// compiler forms the v_and_or_b32 from the expression, as both constants come
+// out of asm statements that it cannot look into.  It must not be an asm
+// statement itself: an MFMA may read a VALU result two wait states after its
+// issue at the earliest, and the compiler inserts those only behind
+// instructions that it knows.  (With v_and_or_b32 as asm, a schedule with one
+// instruction between a pair's word and its MFMA gave wrong sums in one of
+// the four tiles.)
 __device__ __forceinline__ uint32_t nib_pair_k(uint32_t s, uint32_t m, uint32_t c) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(s), "s"(m), "v"(c));
-    return r;
+    return (s & m) | c;
 }
 __device__ __forceinline__ bf16x8_t weight_operand_k(uint32_t word, uint32_t m, uint32_t c) {
     const uint4 q = make_uint4(nib_pair_k(word, m, c), nib_pair_k(word >> 4, m, c), nib_pair_k(word >> 8, m, c),

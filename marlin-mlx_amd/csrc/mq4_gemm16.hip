@@ -135,11 +135,10 @@ __device__ __forceinline__ uint32_t word_of(const uint4& v, int i) {
 
 // (s & m) | c in one v_and_or_b32, the mask in an SGPR and the exponent
 // bits in a VGPR, both set up once by the caller: the nibbles m selects in
-// each 16-bit half as fp16 mantissa bits under c's exponents.
+// each 16-bit half as fp16 mantissa bits under c's exponents.  (Not as asm:
+// see weight_operand_k in mq4_gemm.hip.)
 __device__ __forceinline__ uint32_t nib_pair_h(uint32_t s, uint32_t m, uint32_t c) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(s), "s"(m), "v"(c));
-    return r;
+    return (s & m) | c;
 }
 
 // The eight fp16 weights fp16(s q + b) of one packed word, in the nibble-pair

@@ -1,8 +1,11 @@
 """The build refuses scratch memory in kernels that wait for LDS DMA with exact
 vmcnt counts (marlin-mlx_amd/build.py): the remark parser must find every
-function with a nonzero ScratchSize and nothing else."""
+function with a nonzero ScratchSize and nothing else.  And a rule on the
+sources that the compiler does not check: no VALU arithmetic in asm."""
+import glob
 import importlib.util
 import os
+import re
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -37,3 +40,22 @@ def test_guarded_sources():
     b = _build_module()
     # the two sources whose kernels wait for LDS DMA by exact vmcnt
     assert {"mq4_gemm.hip", "mq4_decode.hip"} <= b.NO_SCRATCH
+
+
+def test_no_vector_arithmetic_in_inline_assembly():
+    """Vector ALU instructions are left to the compiler, which knows the wait
+    states between them and the MFMAs that read their results; behind an asm
+    statement it inserts none.  Constant moves (read by VALU instructions only)
+    are the exception."""
+    csrc = os.path.join(ROOT, "marlin-mlx_amd", "csrc")
+    seen = 0
+    for path in sorted(glob.glob(os.path.join(csrc, "*"))):
+        if not path.endswith((".h", ".hip", ".hpp")):
+            continue
+        with open(path) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        for body in re.findall(r"\basm\b\s*(?:volatile)?\s*\((.*?)\)\s*;", text, re.S):
+            seen += 1
+            ops = re.findall(r"\bv_\w+", body)
+            assert set(ops) <= {"v_mov_b32"}, (os.path.basename(path), body)
+    assert seen >= 10
