@@ -69,11 +69,12 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 // This file is built with MFMA results and accumulators in VGPRs
 // (-amdgpu-mfma-vgpr-form), so the per-group fold reads the MFMA result D
-// directly on the VALU.  The compiler pads each v_mfma_f32_32x32x16_bf16 ->
-// VALU read with 11 wait states, which measured too few on gfx950 (the sums
-// came out wrong); 24 more, once per group between the group's last MFMA and
-// its fold, give the right sums at no measurable cost.  The scheduling
-// barriers keep the padding between the two.
+// directly on the VALU.  The compiler puts the 11 wait states between a
+// v_mfma_f32_32x32x16_bf16 and a VALU read of its result; these 24 more, once
+// per group, are margin only: builds without them give the same bits (K = 320
+// to 6144, both kernels that use them; 3% faster at K = 512).  Wrong sums that
+// were once put down to those 11 came from operands formed in asm statements
+// (weight_operand_k).
 __device__ __forceinline__ void mfma_result_pad() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
@@ -708,9 +709,9 @@ void launch_dma_auto(const GemmArgs& a, hipStream_t st) {
 // address is a constant; scales and biases are read once per eight groups;
 // the next MFMA step's operands are read and formed during the current one;
 // the group's fold waits until the next group's first MFMA step, one tile at
-// a time ahead of the MFMA that overwrites it.  So an MFMA result is read no
-// sooner than 45 instructions after its issue (counted in the built loop),
-// well past the wait states that mfma_result_pad stands for.
+// a time ahead of the MFMA that overwrites it.  The wait states between an
+// MFMA and the VALU read of its result are the compiler's (the read is a plain
+// C++ expression); the schedule leaves 43 instructions there, so it adds none.
 namespace ring {
 
 constexpr int RI = 2, NJ = 2;             // 32 x 32 MFMA tiles of a wave: rows, weight columns
@@ -808,8 +809,7 @@ __global__ __launch_bounds__(64 * WR * WC * KW, 2) void q4_gemm_ring_kernel(Gemm
         bp[t] = reinterpret_cast<const char*>(mat_of(r0).wq) + (int64_t)g0 * 32;
         boff[t] = (uint32_t)((int64_t)wrow_of(r0 + (lane & 31)) * (K / 2) + (lane >> 5) * 16);
     }
-    // scales and biases, 16 bytes (8 groups) of one weight column per lane;
-    // with 64 weight columns one instruction covers gate and up columns
+    // scales and biases, 16 bytes (8 groups) of one weight column per lane
     const char* sbp[SB_I];
     uint32_t sboff[SB_I];
     static_assert(NMAT == 1 || BNW >= 128, "one matrix per scale/bias DMA instruction");

@@ -167,8 +167,8 @@ __device__ __forceinline__ h8_t dequant_word(uint32_t w, h2_t s2, h2_t b2, uint3
 // is r.
 __device__ __forceinline__ int perm8(int r) { return 4 * (r & 1) + (r >> 1); }
 
-// MFMA results are read by the VALU only in the epilogue; the padding keeps
-// the wait states between the last MFMA and that read generous.
+// MFMA results are read by the VALU only in the epilogue; margin on top of the
+// compiler's wait states between the last MFMA and that read.
 __device__ __forceinline__ void mfma_result_pad() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
