@@ -196,10 +196,13 @@ __device__ __forceinline__ uint32_t argmax_key_index(uint64_t key) {
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Wait until at most N vector-memory operations of this wave are outstanding.
+// (The builtin alone orders no memory access for the compiler: the empty asm
+// keeps the reads of data that the wait is for behind it.)
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+    asm volatile("" ::: "memory");
 }
 
 // ---- cross-lane butterfly on the VALU (no LDS round trip) ----

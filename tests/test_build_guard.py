@@ -59,3 +59,13 @@ def test_no_vector_arithmetic_in_inline_assembly():
             ops = re.findall(r"\bv_\w+", body)
             assert set(ops) <= {"v_mov_b32"}, (os.path.basename(path), body)
     assert seen >= 10
+
+
+def test_wait_vmcnt_orders_memory():
+    """The s_waitcnt builtin orders no memory access for the compiler; the
+    helper that every LDS-DMA kernel waits with has to (some read the staged
+    data right after it, with no barrier between)."""
+    with open(os.path.join(ROOT, "marlin-mlx_amd", "csrc", "mq4_device.h")) as f:
+        body = re.search(r"void wait_vmcnt\(\) \{(.*?)\n\}", f.read(), re.S).group(1)
+    after = body.split("__builtin_amdgcn_s_waitcnt", 1)[1]
+    assert 'asm volatile("" ::: "memory")' in after
