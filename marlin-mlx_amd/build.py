@@ -59,9 +59,8 @@ EXTRA_FLAGS = {
 # count assumes no other vector memory traffic in the loop, and register
 # spills to scratch are vector memory operations (a spilling build waits too
 # little and reads stages before their DMA has landed).  The build fails if
-# any kernel in them uses scratch.  (mq4_gemm16.hip waits for all of its
-# DMA every group, but a spilling build would also be a slow one.)
-NO_SCRATCH = {"mq4_gemm.hip", "mq4_gemm16.hip", "mq4_decode.hip"}
+# any kernel in them uses scratch.
+NO_SCRATCH = {"mq4_gemm.hip", "mq4_gemm16.hip", "mq4_decode.hip", "mq4_lmring.hip"}
 
 
 def _scratch_users(remarks: str) -> list[tuple[str, int]]:

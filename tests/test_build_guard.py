@@ -38,8 +38,16 @@ def test_scratch_users_parser():
 
 def test_guarded_sources():
     b = _build_module()
-    # the two sources whose kernels wait for LDS DMA by exact vmcnt
+    # the sources whose kernels wait for LDS DMA by exact vmcnt: those that
+    # call wait_vmcnt with a count above 0
     assert {"mq4_gemm.hip", "mq4_decode.hip"} <= b.NO_SCRATCH
+    csrc = os.path.join(ROOT, "marlin-mlx_amd", "csrc")
+    exact = set()
+    for path in glob.glob(os.path.join(csrc, "*.hip")):
+        with open(path) as f:
+            if re.search(r"\bwait_vmcnt<(?!0>)", f.read()):
+                exact.add(os.path.basename(path))
+    assert exact == b.NO_SCRATCH
 
 
 def test_no_vector_arithmetic_in_inline_assembly():
