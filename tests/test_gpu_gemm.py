@@ -263,14 +263,17 @@ def test_mlp_residual_one_call(mq4, O, dev, M, K, N):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,shift", [(200, "down"), (1960, "down"), (4096, "down"), (200, "gate")])
+@pytest.mark.parametrize("M,shift", [(40, "down"), (128, "down"), (200, "down"), (1960, "down"), (4096, "down"),
+                                     (200, "gate")])
 def test_mlp_residual_paired_down(mq4, O, dev, M, shift):
     """The one-call MLP with one matrix's scales and biases 4-byte but not
     16-byte aligned.  down: gate/up on the fp16-weight GEMM writes h paired
     in bf16 (pair order through the per-chunk column permutation) with its
     group sums from the LDS tile, and the down product runs on the
     exact-operand GEMM (M = 4096: its 64 x 64 wave tiles, 512 blocks of
-    128 x 128; below: 64 x 32).  gate: both products on the exact-operand
+    128 x 128; below: 64 x 32).  M = 40 and 128 take gate/up's 64 x 128 tile,
+    whose two K teams exchange their sums through the LDS that the group sums'
+    tile then uses.  gate: both products on the exact-operand
     GEMM with paired operands.  Against the separate entries: >= 95% of the bits
     identical, rms of the difference <= 1e-2 of the MLP output's rms; against
     the oracle chain on sampled rows: rms(err) <= 1e-2 of that rms."""

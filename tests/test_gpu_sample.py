@@ -221,12 +221,16 @@ def test_infinite_largest_value(mq4, dev, chunked):
     assert keep.all() and np.isinf(S.scaled_logits(bits[:1], 1e-38, np.float32)[0, idx[0]])
 
 
-@pytest.mark.parametrize("M,V", [(1, 8192), (1, 8200), (3, 10248), (1, 151936), (4, 248320), (32, 65536), (128, 8192)])
+@pytest.mark.parametrize("M,V", [(1, 8192), (1, 8200), (3, 10248), (1, 151936), (4, 248320), (6, 248320), (9, 151944),
+                                 (32, 65536), (128, 8192), (128, 8200)])
 def test_candidate_lists_agree_with_single_workgroup(mq4, dev, M, V):
     """Top-k without a keep mask on candidate lists against the one-workgroup
     path, token for token: odd last chunks, ties (more than a list holds, rows of
     one value), infinities, NaN, a row of NaN, the lowest finite value, top_k
-    from 1 past a chunk's size (the chain), with and without top-p."""
+    from 1 past a chunk's size (the chain).  Without top-p the lists run above
+    512 chunks: (128, 8192) is at the line, (6, 248320), (9, 151944), (32,
+    65536) and (128, 8200) are above it, the second and last with an odd last
+    chunk; below it the p = 1.0 entries are the chain's."""
     rng = np.random.default_rng(300 + M + V)
     bits = gen_logits(rng, M, V, "normal")
     bits[-1, : V // 2] = gen_logits(rng, 1, V // 2, "ties")[0]
@@ -317,7 +321,8 @@ def chain_bytes(M, V):
     return 2 * up(8 * mp) + 3 * up(1024 * mp) + 2 * up(2048 * mp) + up(40 * M)
 
 
-@pytest.mark.parametrize("M,V", [(1, 8192), (3, 16392), (32, 248320), (34, 248320), (64, 65536), (128, 8192), (128, 65536)])
+@pytest.mark.parametrize("M,V", [(1, 8192), (3, 16392), (32, 248320), (34, 248320), (64, 65536), (128, 8192),
+                                 (128, 65536)])
 def test_lists_stay_in_the_workspace(mq4, dev, M, V):
     """top_k up to the largest that the lists take, and past it, in a workspace
     of the stated size and in one of the chain's alone (enough for every call;
