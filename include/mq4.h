@@ -120,7 +120,10 @@ int mq4_dequantize(const uint32_t* wq, const uint16_t* scales, const uint16_t* b
  * one bf16 rounding of each output.  Replaces
  * mx::quantized_matmul(x, w, scales, biases, transpose=true, 64, 4)
  * (src/model/marlin.cpp:20-22 and :164-166).  transpose must be 1 (the only
- * form the reference uses).  x and wq must be 16-byte aligned. */
+ * form the reference uses).  x and wq must be 16-byte aligned.  From M = 33
+ * rows on the order of a row's fp32 sums depends on M and N (tiles and K teams
+ * chosen by the number of blocks), so its last bit may differ between calls of
+ * different M. */
 int mq4_qmm(const uint16_t* x, int64_t M, int64_t K,
             const uint32_t* wq, const uint16_t* scales, const uint16_t* biases, int64_t N,
             int transpose, int group_size, int bits, uint16_t* y, void* stream);

@@ -578,7 +578,7 @@ def _process_seed() -> int:
 
 def sample_token(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0, top_p: float = 1.0,
                  seed: int | None = None, return_keep: bool = False):
-    """sample_token (src/sampling/sampler.cpp:9-39) on the GPU, one kernel.
+    """sample_token (src/sampling/sampler.cpp:9-39) on the GPU.
 
     logits: bf16 [1, S, V] (the last position is sampled, as the reference
     slices it) or [M, V] (every row is sampled).  temperature <= 0 is the

@@ -45,9 +45,10 @@
 //    8 groups.
 //  * The ring and the schedule are in gemm16_tile, the tile shapes and the
 //    rule that picks one in tile_for.  At full load (M = 8192) the card holds
-//    the clock at 1.8 GHz (2.6 GHz with few blocks) and MFMAs are busy 57% of
-//    the cycles, as in a large library product (59% at 2.15 GHz): power, not
-//    a unit, is the bound there.
+//    the clock at 1.7-1.8 GHz (2.4 at most) with the socket at 1334 W of its
+//    1400 W cap, and MFMAs are busy 57% of the cycles; a large library product
+//    runs at 1.9-2.0 GHz and 1395 W, 59% busy.  So power management sets the
+//    pace there, and fewer instructions per product are what is left.
 //  * Per 64-k group, the activations (each row's eight 16-byte chunks
 //    XOR-swizzled by (row / 2) % 8: the 16 lanes of a ds_read_b128 phase, 16
 //    rows at one chunk, cover the 64 banks once) and the packed weights (per

@@ -438,10 +438,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const uint16_t* __rest
 //   chunk_mass_lo  the top-p high byte; mass and counts per low byte inside it
 //   chunk_draw     k*, the ties kept, this chunk's earlier ties; Gumbel-max
 //   chunk_final    the row's token from the chunks' best keys
-// Only the stages the parameters need are launched (top-k without a keep
-// mask takes the candidate lists below instead).  The integer sums,
-// thresholds and per-element draws are sample_kernel's, so the two paths give
-// identical tokens and keep masks.
+// Only the stages the parameters need are launched (without a keep mask,
+// top-k with top-p, or top-k alone above 512 chunks, takes the candidate lists
+// below instead).  The integer sums, thresholds and per-element draws are
+// sample_kernel's, so the two paths give identical tokens and keep masks.
 constexpr int kCT = 256;                    // threads per chunk workgroup
 constexpr int kCW = kCT / 64;
 constexpr int kStep = kCT * 8;              // logits per step: one 16-byte load per thread
@@ -857,9 +857,9 @@ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 //               that chunk is read again.
 // Keys, masses, thresholds, tie ranks and draws are sample_kernel's, so the
 // token is the same.  Per call, back to back, one row of 248,320 logits, top-k
-// 50 and top-p 0.9: normal logits 25.2 us, half of them masked 26.5, all but
-// 20 masked 30.5 (-inf) or 33.5 (-1e4), one value throughout 41.5; when a
-// chunk with too many ties sent its row to one workgroup's passes 25.2, 310,
+// 50 and top-p 0.9: normal logits 25.5 us, half of them masked 26.3, all but
+// 20 masked 30.4 (-inf) or 32.7 (-1e4), one value throughout 40.6; when a
+// chunk with too many ties sent its row to one workgroup's passes 25.3, 310,
 // 676 and 1234, on the chain 39.0, 39.9, 43.2 and 46.9.
 constexpr int kListCap = 15360;             // candidates of a row in LDS (120 KB)
 constexpr int64_t kListMinChunks = 512;     // without top-p: chunks of a call above which lists pay

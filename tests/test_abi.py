@@ -240,10 +240,10 @@ def test_mlp_residual_workspace_and_validation(mq4):
     """mq4_mlp_workspace_size: h [M, N] bf16, plus for 5-32 rows the two fp32
     K parts of the down product [2, M, K], and from 33 rows on the paired x
     [M, K], the group sums of x and h and the fp16-weight down product's
-    fp32 K parts [S, M, K] (S of 1, 2, 4 with tiles x S <= 256 CUs, the
-    tiles 128 x 128 while ceil(M / 128) ceil(K / 128) <= 512, else 128 x
-    256; no section for S = 1) and the SwiGLU epilogue's SiLU table (4096
-    bf16), each section 256-byte aligned; the
+    fp32 K parts [S, M, K] (S of 1, 2, 3, 4, 6 with tiles x S <= 256 CUs, the
+    tiles by the rows and the number of blocks; no section for S = 1) and the
+    SwiGLU epilogue's sigmoid table (4096 bf16), each section 256-byte
+    aligned; the
     entry rejects a missing, small or misaligned workspace (and bad shapes)
     before enqueueing anything."""
     L = mq4.lib()
@@ -268,7 +268,7 @@ def test_mlp_residual_workspace_and_validation(mq4):
     assert L.mq4_mlp_workspace_size(M8, K, N) == (up(M8 * N * 2) + up(M8 * K * 2) + up(M8 * K // 64 * 4) +
                                                   up(M8 * N // 64 * 4) + lut)
     # the size for M rows covers every smaller row count, also where the
-    # K-part count drops (512 rows: four parts, 513: two)
+    # K-part count drops (512 rows: four parts, 513: three)
     big = L.mq4_mlp_workspace_size(3000, K, N)
     assert all(L.mq4_mlp_workspace_size(m, K, N) <= big for m in (33, 512, 513, 1024, 1025, 2048, 2049, 3000))
     assert L.mq4_mlp_workspace_size(600, K, N) >= up(4 * 512 * K * 4)

@@ -386,7 +386,7 @@ def test_mlp_residual_split_graph_replay(mq4, O, dev, M):
     """The one-call MLP with its down product in K parts plus a combine,
     captured in a HIP graph: at batched-decode sizes (16, 32: two parts per
     16-row tile, bit for bit the separate entries) and at 200 rows (the
-    fp16-weight GEMM, four parts of 24 groups).  Every replay, with eager work
+    fp16-weight GEMM, six parts of 16 groups).  Every replay, with eager work
     and synchronizations between replays and the workspace overwritten with
     0xFF bytes before each, reproduces the eager call bit for bit, as the
     benches replay it."""
