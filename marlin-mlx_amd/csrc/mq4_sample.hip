@@ -919,6 +919,7 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
     for (int t = 0; t < kListSteps; ++t) {
         // eight equal logits (a masked stretch) in one addition: the additions
         // to one address go one by one
+        if (beg + (int64_t)t * kStep >= end) break;    // block-uniform: past the chunk
         if (flat(t)) each(t, [&](uint32_t k, int e) { if (e == 0) atomicAdd(&hist[k >> kDigitShift], 8u); });
         else each(t, [&](uint32_t k, int) { atomicAdd(&hist[k >> kDigitShift], 1u); });
     }
@@ -930,6 +931,7 @@ __global__ __launch_bounds__(kCT) void topk_list_kernel(ListArgs a) {
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < kListSteps; ++t) {
+        if (beg + (int64_t)t * kStep >= end) break;
         const uint32_t n = flat(t) ? 8u : 1u;
         each(t, [&](uint32_t k, int e) {
             if ((k >> kDigitShift) == hb && (e == 0 || n == 1u)) atomicAdd(&hist[k & ((1u << kDigitShift) - 1u)], n);
