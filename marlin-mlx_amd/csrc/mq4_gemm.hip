@@ -70,16 +70,12 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // This file is built with MFMA results and accumulators in VGPRs
 // (-amdgpu-mfma-vgpr-form), so the per-group fold reads the MFMA result D
 // directly on the VALU.  The compiler puts the 11 wait states between a
-// v_mfma_f32_32x32x16_bf16 and a VALU read of its result; these 24 more, once
-// per group, are margin only: builds without them give the same bits (K = 320
-// to 6144, both kernels that use them; 3% faster at K = 512).  Wrong sums that
-// were once put down to those 11 came from operands formed in asm statements
-// (weight_operand_k).
-__device__ __forceinline__ void mfma_result_pad() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
-    __builtin_amdgcn_sched_barrier(0);
-}
+// v_mfma_f32_32x32x16_bf16 and a VALU read of its result.  (Sums that were
+// once wrong without further ones came from operands formed in asm statements,
+// see weight_operand_k; 24 more per group gave the same bits at 17 shapes, K =
+// 320 to 6144, and cost 2-3% at K = 512.)  The barrier keeps the fold behind
+// the group's last MFMA in the schedule.
+__device__ __forceinline__ void fold_barrier() { __builtin_amdgcn_sched_barrier(0); }
 
 __device__ __forceinline__ bf16x8_t weight_operand(uint32_t word) {
     const uint4 q = make_uint4(nib_pair_bf16<0>(word), nib_pair_bf16<1>(word), nib_pair_bf16<2>(word),
@@ -243,7 +239,7 @@ __global__ __launch_bounds__(kThreads, 2) void q4_gemm_kernel(GemmArgs p) {
                 for (int j = 0; j < 2; ++j)
                     D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], ks == 0 ? zero : D[i][j], 0, 0, 0);
         }
-        mfma_result_pad();
+        fold_barrier();
         // fold the group: acc += s * D + (b - 128 s) * X
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -531,7 +527,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void q4_gemm_dma_kernel(GemmArgs p
                 for (int j = 0; j < TJ; ++j)
                     D[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], ks == 0 ? zero : D[i][j], 0, 0, 0);
         }
-        mfma_result_pad();
+        fold_barrier();
         float X[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -1008,7 +1004,6 @@ __global__ __launch_bounds__(64 * WR * WC * KW, 2) void q4_gemm_ring_kernel(Gemm
         step(std::integral_constant<int, 7>{});
     }
     wait_vmcnt<0>();                                     // no DMA outstanding past the loop
-    mfma_result_pad();
 #pragma unroll
     for (int i = 0; i < RI; ++i)
 #pragma unroll

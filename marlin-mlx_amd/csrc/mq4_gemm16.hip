@@ -168,14 +168,6 @@ __device__ __forceinline__ h8_t dequant_word(uint32_t w, h2_t s2, h2_t b2, uint3
 // is r.
 __device__ __forceinline__ int perm8(int r) { return 4 * (r & 1) + (r >> 1); }
 
-// MFMA results are read by the VALU only in the epilogue; margin on top of the
-// compiler's wait states between the last MFMA and that read.
-__device__ __forceinline__ void mfma_result_pad() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 // One block's tile: rows m0 .. m0 + TBM - 1, weight columns of n0 .., K part
 // kpart of S_K (split again over the block's KW teams).
 template <int EPI, int WR, int WC, int RI, int S, int KW, class Sm>
@@ -416,7 +408,6 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Args& p, Sm& smem_all, i
         step(std::integral_constant<int, 7>{});
     }
     wait_vmcnt<0>();                                 // no DMA outstanding past the loop
-    mfma_result_pad();
 
     // Teams: each takes over OWN of every wave's row tiles, adding the teams'
     // sums in team order; they travel through LDS (the rings, free now), each
